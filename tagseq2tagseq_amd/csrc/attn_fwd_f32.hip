@@ -4,25 +4,13 @@
 // (torch/_higher_order_ops/flex_attention.py:202-267): S = Q K^T * scale,
 // P = softmax of the masked row, O = P V with P kept in float32 (the
 // reference's P.to(dtype) is a no-op for float32), fully masked rows giving
-// O = 0 and LSE = -inf.  Every product and sum is float32
-// (v_mfma_f32_32x32x2_f32).
+// O = 0 and LSE = -inf.  Every product and sum is float32.
 //
-// It walks the same BlockMask lists and tile bitmaps as the bf16 kernel, with
-// the same per-(b, query head, 128-query tile) work-groups, 64-key halves
-// (the bf16 kernel's step at D = 64; its D = 128 form uses 32-key steps)
-// double-buffered in LDS by direct global->LDS copies (a float32 row of D
-// values is copied as a bf16 row of 2 D, so the copy units and row padding
-// are the bf16 ones: pitch D + 4 floats) and lazy-rescaled online softmax in
-// the log2 domain.  What differs is the operand mapping of the 2-deep fp32
-// contraction, chosen so that every operand is a plain row-major LDS read:
-//   S^T = K Q^T, k-step s pairs head dims s and s + D/2 (lane group g takes
-//     d = g D/2 + s), so a lane's K and Q pieces are contiguous; keys in
-//     natural order in the accumulator rows, queries in the lanes.
-//   O^T += V^T P^T, k-step ks of a 32-key block takes the keys of
-//     accumulator entry ks (key acc_row(ks, g) for lane group g), so P^T is
-//     the S^T accumulator entry itself; output row m of tile dt is head dim
-//     DT m + dt, so a lane's V piece for all DT tiles is one contiguous read.
-#include "attn_kernels.h"
+// One work-group per (b, query head, 32 queries), the key blocks dealt to its
+// four waves (attn_f32.h); each wave keeps its own running max, sum and O,
+// merged at the end.  S^T = K Q^T (keys in the accumulator rows, queries in
+// the lanes), lazily rescaled softmax in the log2 domain, O^T += V^T P^T.
+#include "attn_f32.h"
 
 namespace t2t {
 
@@ -39,222 +27,169 @@ struct FwdF32Params {
   MaskTables m;
 };
 
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ f32x16 mfma32_f32(float a, float b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-// Seed of a mixed 32-key block for keys in natural order: 0 where the pair
-// is allowed, -inf where it is masked.  nw = ~w >> (4 g): entry i of lane
-// group g is key acc_row(i, g) = 8 (i / 4) + 4 g + i % 4.
-template <int I = 0>
-__device__ __forceinline__ void mask_seed_fill(f32x16& c, uint32_t nw) {
-  if constexpr (I < 16) {
-    c[I] = __int_as_float(sbfe1_c<8 * (I >> 2) + (I & 3)>(nw) & (int)0xff800000);
-    mask_seed_fill<I + 1>(c, nw);
-  }
-}
-
 }  // namespace
 
 template <int D>
-__global__ __launch_bounds__(kThreads, 1) void attn_fwd_f32_kernel(FwdF32Params p) {
-  constexpr int KS = D / 2;   // MFMA k-steps over the head dim
-  constexpr int DT = D / 32;  // 32-row output tiles
-  constexpr int P = D + 4;    // LDS row pitch (floats)
-  using U = UnitDma<2 * D>;   // a float row of D = a bf16 row of 2 D
-  constexpr int kUnit = U::kRows * P;
-  static_assert(U::kRows * pitch<2 * D>() == 2 * kUnit, "fp32 unit = bf16 unit of 2 D");
-  __shared__ __attribute__((aligned(16))) float k_lo[kUnit], k_hi[kUnit], v_lo[kUnit], v_hi[kUnit];
-  __shared__ __attribute__((aligned(16))) uint32_t bits_lds[2][kTile * 4];
+__global__ __launch_bounds__(kThreads, 3) void attn_fwd_f32_kernel(FwdF32Params p) {
+  constexpr int DT = D / 32;
+  constexpr int P = f32::pitch<D>();
+  // Q rows during the walk, the merge of the four O accumulators after it
+  constexpr int kOwn = f32::kRows * P, kMerge = f32::merge_floats<D>();
+  __shared__ __attribute__((aligned(16))) float lds[kOwn > kMerge ? kOwn : kMerge];
+  __shared__ float stat[2][4][32];  // running max and sum per wave and query
+  __shared__ uint8_t flags[2][4][64];
 
-  const int h = blockIdx.x, b = blockIdx.z;
+  int h, y;
+  head_and_slot(p.Hq, p.Hkv, 4 * p.m.nt, h, y);
+  const int b = blockIdx.z;
   const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = tid & 63;
   const int g = lane >> 5, n = lane & 31;
   const int hk = h / (p.Hq / p.Hkv);
   const int mb = p.m.Bm > 1 ? b : 0;
   const int T = p.T, nt = p.m.nt;
-  const int qt = uniform(p.m.row_order[(size_t)mb * nt + blockIdx.y]);
-  const int q0 = qt * kTile;
-  const int qloc = 32 * wave + n;
-  const int qrow = q0 + qloc;
+  const int qt = uniform(p.m.row_order[(size_t)mb * nt + (y >> 2)]);
+  const int qloc = 32 * (3 - (y & 3)) + n;  // within a tile the later queries see more keys
+  const int qrow = qt * kTile + qloc;
+  if (qrow - n >= T) return;
   const bool qvalid = qrow < T;
   const float c = p.scale_log2;
 
-  // Q^T operand: lane (g, n) holds Q[qrow][g D/2 + s], s = 0 .. D/2 - 1.
-  float qf[KS];
+  // Q rows, requested before the tile list's chain of loads
+  const int srow = tid >> 3, scol = 4 * (tid & 7);
+  f32x4 q4[DT];
   {
-    const float* qp = p.q + b * p.q_sb + h * p.q_sh + (int64_t)(qvalid ? qrow : 0) * p.q_st + g * KS;
+    const float* qb = p.q + b * p.q_sb + h * p.q_sh + (int64_t)(qrow - n + srow) * p.q_st + scol;
 #pragma unroll
-    for (int s = 0; s < KS; s += 4) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(qp + s);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) qf[s + e] = qvalid ? x[e] : 0.f;
+    for (int i = 0; i < DT; ++i) {
+      q4[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (qrow - n + srow < T) q4[i] = *reinterpret_cast<const f32x4*>(qb + 32 * i);
     }
   }
-
-  const float* kbase = p.k + b * p.k_sb + hk * p.k_sh;
-  const float* vbase = p.v + b * p.v_sb + hk * p.v_sh;
-  int koff[U::kPerWave + 1], voff[U::kPerWave + 1];
-#pragma unroll
-  for (int j = 0; j < U::kPerWave; ++j) {
-    koff[j] = unit_dma_offset<2 * D>(wave + kWaves * j, 2 * p.k_st, lane);
-    voff[j] = unit_dma_offset<2 * D>(wave + kWaves * j, 2 * p.v_st, lane);
-  }
-  koff[U::kPerWave] = unit_dma_offset<2 * D>(U::kInsts - 1, 2 * p.k_st, lane);
-  voff[U::kPerWave] = unit_dma_offset<2 * D>(U::kInsts - 1, 2 * p.v_st, lane);
-
   const size_t row = (size_t)mb * nt + qt;
-  const int npart = uniform(p.m.kv_num[row]);
-  const int nfull = uniform(p.m.full_kv_num[row]);
-  const int ntiles = npart + nfull;
-  const int32_t* pidx = p.m.kv_idx + row * nt;
-  const int32_t* fidx = p.m.full_kv_idx + row * nt;
-  const uint32_t* bits_row = p.m.tile_bits + (size_t)p.m.kv_bits_off[row] * kTileBitsWords;
-
-  auto load_chunk = [&](int chunk) {
-    const int it = 64 * chunk + lane;
-    return it < npart ? pidx[it] : (it < ntiles ? fidx[it - npart] : 0);
-  };
-  int tiles_v = load_chunk(0);
-  auto tile_of = [&](int it) { return __builtin_amdgcn_readlane(tiles_v, it & 63); };
-  const auto krs = slice_rsrc(reinterpret_cast<const __bf16*>(kbase), 2 * p.k_st, T, 2 * D);
-  const auto vrs = slice_rsrc(reinterpret_cast<const __bf16*>(vbase), 2 * p.v_st, T, 2 * D);
-  const int k_row4 = (int)p.k_st * 4, v_row4 = (int)p.v_st * 4;
-  // K and V rows [t0, t0 + 64) into one half's units (rows past T read zero).
-  auto load_half = [&](float* kd, float* vd, int t0) {
-    unit_dma<2 * D>(reinterpret_cast<__bf16*>(kd), krs, koff, t0 * k_row4, wave, 0);
-    unit_dma<2 * D>(reinterpret_cast<__bf16*>(vd), vrs, voff, t0 * v_row4, wave, 1);
-  };
-  // bitmap of iteration it: KV tile kt, slot kv_bits_off + kt
-  auto load_bits = [&](int it, int kt) {
-    const bool has = it < npart;
-    const auto rs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint32_t*>(bits_row + (has ? (size_t)kt * kTileBitsWords : 0)), 0,
-        has ? kTile * 16 : 0, 0x00020000);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        rs, (__attribute__((address_space(3))) void*)(&bits_lds[it & 1][(wave & 1) * 256]), 16,
-        (wave & 1) * 1024 + lane * 16, 0, 0, 0);
-  };
+  f32::BlockWalk walk;
+  walk.pidx = p.m.kv_idx + row * nt;
+  walk.fidx = p.m.full_kv_idx + row * nt;
+  walk.pslot = nullptr;
+  walk.words = p.m.tile_bits + (size_t)uniform(p.m.kv_bits_off[row]) * kTileBitsWords;
+  walk.woff = qloc * 4;
+  walk.npart = uniform(p.m.kv_num[row]);
+  walk.ntiles = walk.npart + uniform(p.m.full_kv_num[row]);
+  walk.lane = lane;
+  walk.wave = wave;
+  walk.t0 = 0;
+  walk.cnt = ((y >> 2) + y) & 3;  // no wave, hence no SIMD, always takes the odd blocks
+  walk.look((uint32_t)(qloc - n) * 4);
+  const auto krs = f32::slice(p.k + b * p.k_sb + hk * p.k_sh, p.k_st, T, D);
+  const auto vrs = f32::slice(p.v + b * p.v_sb + hk * p.v_sh, p.v_st, T, D);
+  const int k_st4 = (int)p.k_st * 4, v_st4 = (int)p.v_st * 4;
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+    *reinterpret_cast<f32x4*>(lds + srow * P + scol + 32 * i) = q4[i];
+  walk.publish(flags);
+  __syncthreads();
+  walk.gather(flags);
 
   f32x16 oacc[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) oacc[dt] = f32x16{};
   float m_ref = -INFINITY, l_run = 0.f;
 
-  // One 64-key half (two 32-key blocks j): S^T = K Q^T (+ mask seed),
-  // lazy-rescaled online softmax, O^T += V^T P^T.
-  auto half_step = [&](const float* kt_lds, const float* vt_lds, uint32_t w0, uint32_t w1,
-                       bool partial) {
-    if (partial && __ballot((w0 | w1) != 0u) == 0ull) return;
-    f32x16 st[2];
-    if (partial && __ballot((w0 & w1) != ~0u) != 0ull) {
-      mask_seed_fill(st[0], ~w0 >> (4 * g));
-      mask_seed_fill(st[1], ~w1 >> (4 * g));
-    } else {
-      st[0] = f32x16{};
-      st[1] = f32x16{};
+  // Units of a block: U of K rows (S), 4 of V tokens (P V).
+  constexpr int U = D / 32, NU = U + 4, R = NU % 4 ? 3 : 4;
+  static_assert(NU % R == 0, "a block ends where the ring does");
+  f32x4 x[R][4];  // ring: unit u in slot u % R
+  for (;;) {
+    int base = 0, next;
+    uint32_t w = 0, next_w;
+    bool mixed = false, next_mixed;
+    if (walk.m > 0) {
+      walk.block(0, base, w, mixed);
+      f32::load_row(x[0], krs, (base + n) * k_st4 + 16 * g, 0);
+      f32::load_row(x[1], krs, (base + n) * k_st4 + 16 * g, 1);
     }
+    for (int i = 0; i < walk.m; ++i) {
+      // lane terms are made anew for each block: held across the loop they
+      // would take the kernel past the 168 registers of three waves per SIMD
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      const int g = ln >> 5, n = ln & 31;
+      const float* own = lds + n * P + 4 * g;
+      const int koff = n * k_st4 + 16 * g, voff = 4 * g * v_st4 + 4 * DT * n;
+      f32::OwnPair qx;
+      f32::load_own(qx, own, 0);
+      f32x16 st = {};
+      if (mixed) f32::seed_fill(st, ~w >> (4 * g));
+      // (the last block's successor is itself: its rows are requested to no use)
+      walk.block(min(i + 1, walk.m - 1), next, next_w, next_mixed);
 #pragma unroll
-    for (int s4 = 0; s4 < KS; s4 += 4) {
+      for (int u = 0; u < NU; ++u) {
+        const int a = u + 2;  // unit to request
+        if (a < U) f32::load_row(x[a % R], krs, base * k_st4 + koff, a);
+        else if (a < NU) f32::load_tok<D>(x[a % R], vrs, base * v_st4 + voff, v_st4, a - U);
+        else f32::load_row(x[a % R], krs, next * k_st4 + koff, a - NU);
+        if (u == U) {
+          float mx = st[0];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const f32x4 kf = *reinterpret_cast<const f32x4*>(kt_lds + (32 * j + n) * P + g * KS + s4);
+          for (int e = 1; e < 16; ++e) mx = fmaxf(mx, st[e]);
+          mx = halves_max(mx);
+          const bool move = (mx - m_ref) * c > 8.f;
+          if (__ballot(move) != 0ull) {
+            const float alpha = move ? fast_exp2((m_ref - mx) * c) : 1.f;
+            l_run *= alpha;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) st[j] = mfma32_f32(kf[e], qf[s4 + e], st[j]);
-      }
-    }
-    float mx = -INFINITY;
+            for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;
+            m_ref = move ? mx : m_ref;
+          }
+          const float neg = m_ref == -INFINITY ? 0.f : -m_ref * c;
+          float rs = 0.f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[j][i]);
-    mx = halves_max(mx);
-    const bool move = (mx - m_ref) * c > 8.f;
-    if (__ballot(move) != 0ull) {
-      const float alpha = move ? fast_exp2((m_ref - mx) * c) : 1.f;
-      l_run *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;
-      m_ref = move ? mx : m_ref;
-    }
-    const float neg = m_ref == -INFINITY ? 0.f : -m_ref * c;
-    float rs = 0.f;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        st[j][i] = fast_exp2(fmaf(st[j][i], c, neg));
-        rs += st[j][i];
-      }
-    l_run += halves_sum(rs);
-    // O^T += V^T P^T: k-step ks of block j takes key 32 j + acc_row(ks, g).
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int ks = 0; ks < 16; ++ks) {
-        const float* vr = vt_lds + (32 * j + acc_row(ks, g)) * P + DT * n;
-        if constexpr (DT == 4) {
-          const f32x4 vf = *reinterpret_cast<const f32x4*>(vr);
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) oacc[dt] = mfma32_f32(vf[dt], st[j][ks], oacc[dt]);
-        } else {
-          const f32x2 vf = *reinterpret_cast<const f32x2*>(vr);
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) oacc[dt] = mfma32_f32(vf[dt], st[j][ks], oacc[dt]);
+          for (int e = 0; e < 16; ++e) {
+            st[e] = fast_exp2(fmaf(st[e], c, neg));
+            rs += st[e];
+          }
+          l_run += rs;  // over the lane's own half of the keys
         }
+        f32::fence();
+        if (u < U) f32::dot_unit(st, x[u % R], qx, own, u == U - 1 ? own : nullptr, u);
+        else f32::acc_unit<D>(oacc, x[u % R], st, u - U);
+        f32::fence();
       }
-  };
-
-  int k0_next = ntiles > 0 ? tile_of(0) * kTile : 0;
-  if (ntiles > 0) {
-    load_half(k_lo, v_lo, k0_next);
-    if (npart > 0) load_bits(0, k0_next / kTile);
-  }
-  for (int it = 0; it < ntiles; ++it) {
-    const bool partial = it < npart;
-    const int k0 = k0_next;
-    dma_barrier();
-    uint4 mbits = make_uint4(~0u, ~0u, ~0u, ~0u);
-    if (partial) mbits = *reinterpret_cast<const uint4*>(&bits_lds[it & 1][qloc * 4]);
-    load_half(k_hi, v_hi, k0 + 64);
-    half_step(k_lo, v_lo, mbits.x, mbits.y, partial);
-
-    dma_barrier();
-    const bool more = it + 1 < ntiles;
-    if (more) {
-      if (((it + 1) & 63) == 0) tiles_v = load_chunk((it + 1) >> 6);
-      k0_next = tile_of(it + 1) * kTile;
-      load_half(k_lo, v_lo, k0_next);
-      load_bits(it + 1, k0_next / kTile);
+      base = next;
+      w = next_w;
+      mixed = next_mixed;
     }
-    half_step(k_hi, v_hi, mbits.z, mbits.w, partial);
+    if (walk.t0 >= walk.ntiles) break;
+    walk.look((uint32_t)(qloc - n) * 4);
+    walk.publish(flags);
+    __syncthreads();
+    walk.gather(flags);
   }
 
-  if (qvalid) {
-    const float inv_l = l_run > 0.f ? 1.f / l_run : 0.f;
-    float* op = p.o + b * p.o_sb + h * p.o_sh + (int64_t)qrow * p.o_st;
-    // Output row m of tile dt is head dim DT m + dt.
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int d0 = DT * acc_row(i, g);
-      if constexpr (DT == 4) {
-        f32x4 w;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) w[dt] = oacc[dt][i] * inv_l;
-        *reinterpret_cast<f32x4*>(op + d0) = w;
-      } else {
-        f32x2 w;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) w[dt] = oacc[dt][i] * inv_l;
-        *reinterpret_cast<f32x2*>(op + d0) = w;
-      }
-    }
-    if (g == 0)
-      p.lse2[((size_t)b * p.Hq + h) * T + qrow] =
-          l_run > 0.f ? m_ref * c + __log2f(l_run) : -INFINITY;
+  // Merge: each wave's O and sum brought to the largest running max.
+  l_run = halves_sum(l_run);
+  if (g == 0) {
+    stat[0][wave][n] = m_ref;
+    stat[1][wave][n] = l_run;
   }
+  __syncthreads();  // Q rows are no longer read either
+  float m_all = stat[0][0][n];
+#pragma unroll
+  for (int u = 1; u < 4; ++u) m_all = fmaxf(m_all, stat[0][u][n]);
+  float l_all = 0.f;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const float mu = stat[0][u][n];  // -inf: the wave saw no allowed pair of this query
+    if (mu != -INFINITY) l_all += stat[1][u][n] * fast_exp2((mu - m_all) * c);
+  }
+  const float alpha = m_ref == -INFINITY ? 0.f : fast_exp2((m_ref - m_all) * c);
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;
+  const float inv_l = l_all > 0.f ? 1.f / l_all : 0.f;
+  f32::merge_store<D>(lds, oacc, inv_l, p.o + b * p.o_sb + h * p.o_sh + (int64_t)qrow * p.o_st,
+                      qvalid, wave, lane);
+  if (qvalid && tid < 32)
+    p.lse2[((size_t)b * p.Hq + h) * T + qrow] =
+        l_all > 0.f ? m_all * c + __log2f(l_all) : -INFINITY;
 }
 
 hipError_t launch_attn_fwd_f32(const TensorView& q, const TensorView& k, const TensorView& v,
@@ -270,7 +205,7 @@ hipError_t launch_attn_fwd_f32(const TensorView& q, const TensorView& k, const T
   p.scale_log2 = dims.scale * kLog2e;
   p.m = mask;
   if (mask.nt == 0 || dims.B == 0 || dims.Hq == 0) return hipSuccess;
-  dim3 grid(dims.Hq, mask.nt, dims.B);
+  dim3 grid(dims.Hq, 4 * mask.nt, dims.B);
   if (dims.D == 64)
     hipLaunchKernelGGL(attn_fwd_f32_kernel<64>, grid, dim3(kThreads), 0, stream, p);
   else
