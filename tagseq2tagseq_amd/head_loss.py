@@ -60,15 +60,19 @@ def _head_pass(x, weight, targets, ignore_index: int, chunk: Optional[int], grad
         raise ValueError(f"{t.numel()} targets for {N} rows")
     if weight.shape[1] != D:
         raise ValueError(f"weight {tuple(weight.shape)} does not match rows of width {D}")
-    w = torch.zeros((ld, D), dtype=torch.bfloat16, device=dev)
-    w[:V].copy_(weight)
+    if ld == V and weight.dtype == torch.bfloat16 and weight.is_contiguous():
+        w = weight.detach()
+    else:
+        w = torch.empty((ld, D), dtype=torch.bfloat16, device=dev)
+        w[:V].copy_(weight)
+        w[V:].zero_()
     n = (t != ignore_index).sum()
     # gradient scale 1 / n; with every row ignored no row has a gradient, so
     # the scale only has to be finite
     scale = (1.0 / n.clamp(min=1).to(torch.float32)).reshape(1)
     row_loss = torch.empty((N,), dtype=torch.float32, device=dev)
     dx = torch.empty((N, D), dtype=x.dtype, device=dev) if grads else None
-    dw = torch.zeros((ld, D), dtype=torch.float32, device=dev) if grads else None
+    dw = None
     if chunk is None:
         chunk = max(1, AUTO_CHUNK_BYTES // (2 * ld))
     rows = max(1, min(chunk, N))
@@ -87,7 +91,10 @@ def _head_pass(x, weight, targets, ignore_index: int, chunk: Optional[int], grad
             _lib.check(rc, "t2t_ce_rows")
             if grads:
                 torch.mm(logits, w, out=dx[r0:r0 + m])
-                dw += _mm_f32(logits.t(), xs)
+                part = _mm_f32(logits.t(), xs)
+                dw = part if dw is None else dw.add_(part)
+    if grads and dw is None:  # no rows
+        dw = torch.zeros((ld, D), dtype=torch.float32, device=dev)
     return row_loss, n, dx, dw
 
 

@@ -65,6 +65,35 @@ def test_ce_rows_against_float64(rows, V, ld):
     assert torch.equal(loss2, loss) and torch.equal(inplace, grad)
 
 
+@pytest.mark.parametrize("V", [2041, 8192, 8193, 16391, 24577, 33000, 40961, 49160, 57345,
+                               65521])
+def test_ce_rows_widths_held_in_registers(V):
+    """Every register count of the one-read kernel, the first and last width that
+    it takes (ld 2048 and 65536), targets in the first and last column, padding that
+    holds infinities, and rows of the type's lowest value and of -inf but for
+    one logit."""
+    ld = (V + 15) // 8 * 8
+    g = torch.Generator(device=DEV).manual_seed(V)
+    x = (torch.randn(6, ld, generator=g, device=DEV) * 3).to(torch.bfloat16)
+    x[:, V:] = float("inf")
+    x[4, :V] = torch.finfo(torch.bfloat16).min
+    x[4, 7] = 1.0
+    x[5, :V] = float("-inf")
+    x[5, V - 1] = 2.0
+    t = torch.tensor([0, V - 1, -100, V // 2, 3, V - 1], device=DEV)
+    loss, grad = _ce_rows(x.clone(), V, t, -100, 0.25)
+    xf = x[:, :V].double()
+    ref = torch.logsumexp(xf, 1) - xf.gather(1, t.clamp(min=0)[:, None])[:, 0]
+    ref[2] = 0
+    torch.testing.assert_close(loss.double(), ref, rtol=1e-5, atol=1e-5)
+    p = torch.softmax(xf, 1)
+    p[torch.arange(6, device=DEV), t.clamp(min=0)] -= 1.0
+    p[2] = 0
+    # one bf16 rounding of the gradient
+    torch.testing.assert_close(grad[:, :V].double(), p * 0.25, rtol=8e-3, atol=1e-6)
+    assert (grad[:, V:] == 0).all() and torch.isfinite(grad).all()
+
+
 def test_ce_rows_out_of_range_target_is_nan():
     x = torch.randn(3, 16, device=DEV).to(torch.bfloat16)
     t = torch.tensor([2, 16, -5], device=DEV)
