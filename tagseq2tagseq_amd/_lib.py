@@ -10,6 +10,9 @@ import os
 import re
 from typing import List
 
+import torch
+from torch.autograd import forward_ad
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libt2t_attn.so")
 HEADER_PATH = os.path.join(os.path.dirname(HERE), "include", "t2t_attn.h")
@@ -39,6 +42,7 @@ class T2TBlockMaskC(ctypes.Structure):
 
 
 _lib = None
+_host = None
 
 _P = ctypes.c_void_p
 _I32 = ctypes.c_int32
@@ -101,6 +105,30 @@ def lib() -> ctypes.CDLL:
             fn.restype = res
         _lib = l
     return _lib
+
+
+def host():
+    """The C++ host side of the per-layer calls (csrc/host_ops.cpp); like the
+    kernels it has no fallback."""
+    global _host
+    if _host is None:
+        lib()  # a library that is missing is reported as such
+        try:
+            from . import _t2t_host
+        except ImportError as e:
+            raise RuntimeError(f"_t2t_host.so is not built or cannot be loaded ({e}); run "
+                               "`python -m tagseq2tagseq_amd.build`") from e
+        _host = _t2t_host
+    return _host
+
+
+def unwatched(*tensors) -> bool:
+    """True when nothing can be watching a call on these tensors -- no graph
+    to record, no forward-mode level, no function transform -- so that it may
+    go to the kernels without an autograd.Function."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    return forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
 
 
 def check(rc: int, what: str) -> None:

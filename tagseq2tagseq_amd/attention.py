@@ -123,39 +123,14 @@ def _mask_struct(block_mask):
 def attn_fwd(q, k, v, block_mask, scale: float):
     """Kernel call: returns (out [B,Hq,T,D] in q.dtype, lse2 float32 [B,Hq,T]).
     ``block_mask``: a T2TBlockMask or its ``tables()`` list."""
-    B, Hq, Hkv, T, D = q.shape[0], q.shape[1], k.shape[1], q.shape[2], q.shape[3]
-    # [B, T, Hq, D] storage seen as [B, Hq, T, D]: the module's output
-    # projection then reads token rows without a transpose copy.
-    out = torch.empty((B, T, Hq, D), dtype=q.dtype, device=q.device).transpose(1, 2)
-    lse2 = torch.empty((B, Hq, T), dtype=torch.float32, device=q.device)
-    qs, ks, vs, os_ = _view(q), _view(k), _view(v), _view(out)
-    with torch.cuda.device(q.device):
-        rc = _lib.lib().t2t_attn_fwd(ctypes.byref(qs), ctypes.byref(ks), ctypes.byref(vs),
-                                     ctypes.byref(os_), lse2.data_ptr(), B, Hq, Hkv, T, D,
-                                     _DTYPE_CODES[q.dtype], float(scale),
-                                     ctypes.byref(_mask_struct(block_mask)), _stream_ptr(q))
-    _lib.check(rc, "t2t_attn_fwd")
-    return out, lse2
+    mask = _mask_struct(block_mask)  # alive until the launch has read it
+    return _lib.host().attn_fwd(q, k, v, ctypes.addressof(mask), scale)
 
 
 def attn_bwd(q, k, v, out, dout, lse2, block_mask, scale: float):
     """Kernel call: returns (dq, dk, dv).  ``block_mask`` as in attn_fwd."""
-    B, Hq, Hkv, T, D = q.shape[0], q.shape[1], k.shape[1], q.shape[2], q.shape[3]
-    if dout.stride(3) != 1:
-        dout = dout.contiguous()
-    dq = torch.empty_like(q, memory_format=torch.contiguous_format)
-    dk = torch.empty_like(k, memory_format=torch.contiguous_format)
-    dv = torch.empty_like(v, memory_format=torch.contiguous_format)
-    delta = torch.empty((B, Hq, T), dtype=torch.float32, device=q.device)
-    views = [_view(t) for t in (q, k, v, out, dout)]
-    gviews = [_view(t) for t in (dq, dk, dv)]
-    with torch.cuda.device(q.device):
-        rc = _lib.lib().t2t_attn_bwd(*[ctypes.byref(x) for x in views], lse2.data_ptr(),
-                                     delta.data_ptr(), *[ctypes.byref(x) for x in gviews],
-                                     B, Hq, Hkv, T, D, _DTYPE_CODES[q.dtype], float(scale),
-                                     ctypes.byref(_mask_struct(block_mask)), _stream_ptr(q))
-    _lib.check(rc, "t2t_attn_bwd")
-    return dq, dk, dv
+    mask = _mask_struct(block_mask)
+    return _lib.host().attn_bwd(q, k, v, out, dout, lse2, ctypes.addressof(mask), scale)
 
 
 class BwdPhases:
@@ -312,6 +287,8 @@ def flex_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
     if torch.compiler.is_compiling():
         # compiled graphs trace the custom op (schema + fake implementation)
         out, lse2 = masked_attention(query, key, value, block_mask.tables(), float(scale))
+    elif _lib.unwatched(query, key, value):
+        out, lse2 = attn_fwd(query, key, value, block_mask, float(scale))
     else:
         # eager: the same kernels through a plain autograd.Function, whose host
         # cost per call is a fraction of the custom op's registered autograd

@@ -21,7 +21,6 @@ evaluated from its ``mask_mod``.
 """
 from __future__ import annotations
 
-import ctypes
 from dataclasses import dataclass, field
 from typing import Callable, Optional
 
@@ -196,37 +195,14 @@ def build_block_mask(doc_ids: torch.Tensor, q_bits: Optional[torch.Tensor] = Non
     W = qb.shape[1]
     if W > _lib.MAX_WORDS:
         raise ValueError(f"{W} grant words exceed the supported {_lib.MAX_WORDS}")
-    nt = (T + TILE - 1) // TILE
-    i32 = dict(dtype=torch.int32, device=device)
-    tile_class = torch.empty((Bm, nt, nt), dtype=torch.int8, device=device)
-    t = {}
-    for name in ("kv", "full_kv", "q", "full_q"):
-        t[name + "_num"] = torch.empty((Bm, 1, nt), **i32)
-        t[name + "_idx"] = torch.empty((Bm, 1, nt, nt), **i32)
-    row_order = torch.empty((Bm, nt), **i32)
-    col_order = torch.empty((Bm, nt), **i32)
-    kv_bits_off = torch.empty((Bm, nt), **i32)
-    q_bits_slot = torch.empty((Bm, nt, nt), **i32)
-    slots = max(1, Bm * nt * (nt + 1) // 2)
-    tile_bits = torch.empty((slots, 2, TILE, 4), **i32)
-    tabs = (t["kv_num"], t["kv_idx"], t["full_kv_num"], t["full_kv_idx"], t["q_num"], t["q_idx"],
-            t["full_q_num"], t["full_q_idx"], row_order, col_order, kv_bits_off, q_bits_slot,
-            tile_bits)
-    cs = tables_c_struct(tabs)
-    s = stream if stream is not None else torch.cuda.current_stream(device)
-    with torch.cuda.device(device):
-        rc = _lib.lib().t2t_mask_meta(
-            doc_ids.data_ptr(), qb.data_ptr() if W else None, kb.data_ptr() if W else None,
-            Bm, T, W, tile_class.data_ptr(), ctypes.byref(cs), ctypes.c_void_p(s.cuda_stream))
-    _lib.check(rc, "t2t_mask_meta")
+    host = _lib.host()
+    s = stream.cuda_stream if stream is not None else host.current_stream(device.index)
+    tile_class, *t = host.mask_meta(doc_ids, qb, kb, s)
     return T2TBlockMask(
         seq_len=T, doc_ids=doc_ids, q_bits=qb, kv_bits=kb, tile_class=tile_class,
-        kv_num_blocks=t["kv_num"], kv_indices=t["kv_idx"],
-        full_kv_num_blocks=t["full_kv_num"], full_kv_indices=t["full_kv_idx"],
-        q_num_blocks=t["q_num"], q_indices=t["q_idx"],
-        full_q_num_blocks=t["full_q_num"], full_q_indices=t["full_q_idx"],
-        row_order=row_order, col_order=col_order, kv_bits_off=kv_bits_off,
-        q_bits_slot=q_bits_slot, tile_bits=tile_bits, _c=cs)
+        **dict(zip(("kv_num_blocks", "kv_indices", "full_kv_num_blocks", "full_kv_indices",
+                    "q_num_blocks", "q_indices", "full_q_num_blocks", "full_q_indices",
+                    "row_order", "col_order", "kv_bits_off", "q_bits_slot", "tile_bits"), t)))
 
 
 def _ordered(flags: torch.Tensor):

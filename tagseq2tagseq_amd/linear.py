@@ -12,15 +12,13 @@ work-groups into fp32 partials and sums them in a fixed order.
 """
 from __future__ import annotations
 
-import ctypes
-
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _lib
 
-_OUT_DTYPE = {torch.bfloat16: 0, torch.float32: 1}
+_OUT_F32 = {torch.bfloat16: False, torch.float32: True}
 
 
 def wgrad_applies(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -28,31 +26,13 @@ def wgrad_applies(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor) -> bo
     M, N = weight.shape
     K = x.numel() // max(N, 1)
     return (x.is_cuda and x.dtype == torch.bfloat16 and dy.dtype == torch.bfloat16
-            and weight.dtype in _OUT_DTYPE and M % 128 == 0 and N % 128 == 0
+            and weight.dtype in _OUT_F32 and M % 128 == 0 and N % 128 == 0
             and K > 0 and K % 64 == 0)
-
-
-def _rows(t: torch.Tensor) -> torch.Tensor:
-    t = t.reshape(-1, t.shape[-1])
-    ok = t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
-    return t if ok else t.contiguous()
 
 
 def wgrad(dy: torch.Tensor, x: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     """dY^T X of [K, M] and [K, N] bf16 rows -> [M, N] (out_dtype)."""
-    d2, x2 = _rows(dy), _rows(x)
-    K, M = d2.shape
-    N = x2.shape[1]
-    L = _lib.lib()
-    ws = torch.empty((L.t2t_wgrad_workspace(M, N, K),), dtype=torch.uint8, device=x.device)
-    out = torch.empty((M, N), dtype=out_dtype, device=x.device)
-    stream = ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
-    with torch.cuda.device(x.device):
-        rc = L.t2t_wgrad(d2.data_ptr(), d2.stride(0), x2.data_ptr(), x2.stride(0),
-                         out.data_ptr(), _OUT_DTYPE[out_dtype], M, N, K, ws.data_ptr(),
-                         ws.numel(), stream)
-    _lib.check(rc, "t2t_wgrad")
-    return out
+    return _lib.host().wgrad(dy, x, _OUT_F32[out_dtype])
 
 
 class WGradLinearFn(torch.autograd.Function):
@@ -86,6 +66,7 @@ class Linear(nn.Linear):
         # (graphs being compiled keep torch's own linear: the Function's
         # backward calls the library through ctypes)
         if (self.bias is None and x.is_cuda and x.dtype == torch.bfloat16
-                and self.weight.dtype == torch.bfloat16 and not torch.compiler.is_compiling()):
+                and self.weight.dtype == torch.bfloat16 and not torch.compiler.is_compiling()
+                and not _lib.unwatched(x, self.weight)):
             return WGradLinearFn.apply(x, self.weight)
         return super().forward(x)

@@ -30,7 +30,7 @@ import torch.utils.checkpoint
 
 from . import norm
 from .attention import FlexSelfAttention
-from .glu import SwiGLUFn, swiglu_applies
+from .glu import swiglu_applies, swiglu_rows
 from .head_loss import HeadCEFn, fused_head_applies, head_loss_needs_grad, head_loss_value
 from .linear import Linear
 
@@ -69,7 +69,7 @@ class GLU(nn.Module):
         gu = self.gate_up(x)
         if self.act is F.silu and swiglu_applies(gu) and not torch.compiler.is_compiling():
             # one fused pass each way (t2t_swiglu), the gradient of [g | u] whole
-            return self.dropout(self.down(SwiGLUFn.apply(gu)))
+            return self.dropout(self.down(swiglu_rows(gu)))
         g, u = gu.chunk(2, dim=-1)
         return self.dropout(self.down(self.act(g) * u))
 

@@ -10,7 +10,6 @@ the weight gradient reduced across work-groups in a fixed order).
 """
 from __future__ import annotations
 
-import ctypes
 from typing import Tuple
 
 import torch
@@ -20,28 +19,8 @@ from . import _lib
 _WDT = {torch.bfloat16: 0, torch.float32: 1}
 
 
-def _stream_ptr(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
-
-
-def _rows(t: torch.Tensor) -> torch.Tensor:
-    t = t.reshape(-1, t.shape[-1])
-    return t if t.stride(1) == 1 and t.stride(0) % 8 == 0 else t.contiguous()
-
-
 def _fwd_impl(x, weight, eps):
-    C = x.shape[-1]
-    xr = _rows(x)
-    N = xr.shape[0]
-    y = torch.empty((N, C), dtype=x.dtype, device=x.device)
-    rstd = torch.empty((N,), dtype=torch.float32, device=x.device)
-    w = weight.contiguous()
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().t2t_rms_norm(xr.data_ptr(), xr.stride(0), w.data_ptr(), _WDT[w.dtype],
-                                     y.data_ptr(), y.stride(0), rstd.data_ptr(), N, C,
-                                     float(eps), _stream_ptr(x))
-    _lib.check(rc, "t2t_rms_norm")
-    return y.view(x.shape), rstd
+    return _lib.host().rms_norm(x, weight, eps)
 
 
 @torch.library.custom_op("t2t::rms_norm", mutates_args=())
@@ -58,22 +37,7 @@ def _rms_norm_fake(x, weight, eps):
 
 
 def _bwd_impl(dy, x, weight, rstd):
-    C = x.shape[-1]
-    xr, dyr = _rows(x), _rows(dy)
-    N = xr.shape[0]
-    dx = torch.empty((N, C), dtype=x.dtype, device=x.device)
-    w = weight.contiguous()
-    dw = torch.empty_like(w)
-    L = _lib.lib()
-    ws = torch.empty(max(1, L.t2t_rms_norm_backward_workspace(N, C) // 4), dtype=torch.float32,
-                     device=x.device)
-    with torch.cuda.device(x.device):
-        rc = L.t2t_rms_norm_backward(dyr.data_ptr(), dyr.stride(0), xr.data_ptr(), xr.stride(0),
-                                     w.data_ptr(), _WDT[w.dtype], rstd.data_ptr(), dx.data_ptr(),
-                                     dx.stride(0), dw.data_ptr(), ws.data_ptr(), ws.numel() * 4,
-                                     N, C, _stream_ptr(x))
-    _lib.check(rc, "t2t_rms_norm_backward")
-    return dx.view(x.shape), dw
+    return _lib.host().rms_norm_backward(dy, x, weight, rstd)
 
 
 @torch.library.custom_op("t2t::rms_norm_backward", mutates_args=())
@@ -132,4 +96,6 @@ class RMSNormFn(torch.autograd.Function):
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     if torch.compiler.is_compiling():
         return rms_norm_op(x, weight, float(eps))[0]
+    if _lib.unwatched(x, weight):
+        return _fwd_impl(x, weight, float(eps))[0]
     return RMSNormFn.apply(x, weight, float(eps))

@@ -15,7 +15,6 @@ Kernels: libt2t_attn.so ``t2t_qkv_rope`` / ``t2t_qkv_rope_backward``.
 """
 from __future__ import annotations
 
-import ctypes
 from typing import Dict, Tuple
 
 import torch
@@ -23,10 +22,6 @@ import torch
 from . import _lib
 
 _TABLES: Dict[Tuple[int, int, float, str], Tuple[torch.Tensor, torch.Tensor]] = {}
-
-
-def _stream_ptr(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
 
 
 def rope_tables(head_dim: int, rows: int, device, base: float = 10000.0):
@@ -51,38 +46,11 @@ def _split_dims(qkv: torch.Tensor, num_heads: int):
 
 
 def _qkv_rope_impl(qkv, cos, sin, num_heads, pos0):
-    B, T, D = _split_dims(qkv, num_heads)
-    H = num_heads
-    if qkv.dtype != torch.bfloat16:
-        raise NotImplementedError(f"qkv dtype {qkv.dtype} is not supported (bfloat16 only)")
-    if not qkv.is_cuda:
-        raise RuntimeError("the prologue kernel needs ROCm GPU tensors")
-    if qkv.stride(2) != 1:
-        qkv = qkv.contiguous()
-    cos, sin = cos.contiguous(), sin.contiguous()
-    q, k, v = (torch.empty((B, H, T, D), dtype=qkv.dtype, device=qkv.device) for _ in range(3))
-    views = [_lib.tensor_struct(t) for t in (q, k, v)]
-    with torch.cuda.device(qkv.device):
-        rc = _lib.lib().t2t_qkv_rope(qkv.data_ptr(), qkv.stride(0), qkv.stride(1), B, T, H, D,
-                                     cos.data_ptr(), sin.data_ptr(), cos.shape[0], pos0,
-                                     *[ctypes.byref(x) for x in views], _stream_ptr(qkv))
-    _lib.check(rc, "t2t_qkv_rope")
-    return q, k, v
+    return _lib.host().qkv_rope(qkv, cos, sin, num_heads, pos0)
 
 
 def _qkv_rope_bwd_impl(dq, dk, dv, cos, sin, pos0):
-    B, H, T, D = dq.shape
-    grads = [g if g.stride(3) == 1 else g.contiguous() for g in (dq, dk, dv)]
-    cos, sin = cos.contiguous(), sin.contiguous()
-    dqkv = torch.empty((B, T, 3 * H * D), dtype=dq.dtype, device=dq.device)
-    views = [_lib.tensor_struct(g) for g in grads]
-    with torch.cuda.device(dq.device):
-        rc = _lib.lib().t2t_qkv_rope_backward(*[ctypes.byref(x) for x in views], cos.data_ptr(),
-                                              sin.data_ptr(), cos.shape[0], pos0, B, T, H, D,
-                                              dqkv.data_ptr(), dqkv.stride(0), dqkv.stride(1),
-                                              _stream_ptr(dq))
-    _lib.check(rc, "t2t_qkv_rope_backward")
-    return dqkv
+    return _lib.host().qkv_rope_backward(dq, dk, dv, cos, sin, pos0)
 
 
 @torch.library.custom_op("t2t::qkv_rope", mutates_args=())
@@ -169,4 +137,6 @@ def qkv_rope(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, num_heads:
         return qkv_rope_torch(qkv, cos, sin, num_heads, pos0)
     if torch.compiler.is_compiling():
         return qkv_rope_op(qkv, cos, sin, int(num_heads), int(pos0))
+    if _lib.unwatched(qkv, cos, sin):
+        return _qkv_rope_impl(qkv, cos, sin, int(num_heads), int(pos0))
     return QKVRopeFn.apply(qkv, cos, sin, int(num_heads), int(pos0))
