@@ -396,6 +396,18 @@ int t2t_first_input_diff(const int64_t *tokens_a, const int64_t *tokens_b, const
                          int32_t *out, void *stream);
 
 /*
+ * Linear map of bf16 token rows, fp32 sums, rounded once: y [M][N] = x [M][K]
+ * W^T with W [N][K] (w_transposed 0: a projection's forward, F.linear without
+ * bias), or x W with W [K][N] (w_transposed 1: its input gradient).  For the
+ * layers' projections (model/modules/layer.py:33-35) of up to a few thousand
+ * tokens.  K and W's row length are multiples of 8, x and w 16-byte aligned
+ * with strides (elements) multiples of 8, each under 2 GiB; y any alignment.
+ */
+int t2t_linear(const void *x, int64_t x_stride, const void *w, int64_t w_stride,
+               int32_t w_transposed, void *y, int64_t y_stride, int32_t M, int32_t N, int32_t K,
+               void *stream);
+
+/*
  * Weight gradient of a linear map over many rows: C[m][n] = sum over k of
  * A[k][m] B[k][n], i.e. dW = dY^T X for y = x W^T with dY [K][M] and X [K][N].
  * Replaces the weight-gradient product of nn.Linear's backward for the

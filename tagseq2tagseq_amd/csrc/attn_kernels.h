@@ -121,6 +121,12 @@ int wgrad_splits(int M, int N, int K);
 hipError_t launch_wgrad(const __bf16* a, int64_t lda, const __bf16* b, int64_t ldb, float* part,
                         void* out, bool out_f32, int M, int N, int K, hipStream_t stream);
 
+// Linear maps of a short sequence: y = x W^T (nn false: W [N][K]) or y = x W
+// (nn true: W [K][N]); K a multiple of 8, rows 16-byte aligned, each operand
+// under 2 GiB.
+hipError_t launch_linear(bool nn, const __bf16* x, int64_t xs, const __bf16* w, int64_t ws,
+                         __bf16* y, int64_t ys, int M, int N, int K, hipStream_t stream);
+
 // SwiGLU: h = silu(g) u from [g | u] rows, and [dg | du] from dh.
 hipError_t launch_swiglu_fwd(const __bf16* gu, int64_t gs, __bf16* h, int64_t hs, int N, int H,
                              hipStream_t stream);

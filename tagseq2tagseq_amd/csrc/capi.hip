@@ -504,6 +504,32 @@ int t2t_rms_norm(const void* x, int64_t x_stride, const void* weight, int32_t we
                     "t2t_rms_norm launch");
 }
 
+int t2t_linear(const void* x, int64_t x_stride, const void* w, int64_t w_stride,
+               int32_t w_transposed, void* y, int64_t y_stride, int32_t M, int32_t N, int32_t K,
+               void* stream) {
+  if (M < 0 || N < 0 || K <= 0) return fail(T2T_EINVAL, "M=%d N=%d K=%d", M, N, K);
+  if (M == 0 || N == 0) return T2T_OK;
+  const int64_t w_rows = w_transposed ? K : N, w_cols = w_transposed ? N : K;
+  if (K % 8 || w_cols % 8)
+    return fail(T2T_EUNSUPPORTED, "rows of %d and %lld elements: multiples of 8 needed", K,
+                (long long)w_cols);
+  if (!x || !w || !y) return fail(T2T_EINVAL, "x / w / y is NULL");
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15)
+    return fail(T2T_EINVAL, "x and w must be 16-byte aligned");
+  if (x_stride % 8 || w_stride % 8 || x_stride < K || w_stride < w_cols || y_stride < N)
+    return fail(T2T_EINVAL, "row strides %lld, %lld, %lld", (long long)x_stride,
+                (long long)w_stride, (long long)y_stride);
+  // the copies address an operand, and up to a tile past it, with 31-bit offsets
+  const int64_t limit = 0x7ffffff0LL;
+  if (((int64_t)M + 128) * x_stride * 2 > limit || (w_rows + 128) * w_stride * 2 > limit)
+    return fail(T2T_EUNSUPPORTED, "an operand of 2 GiB or more");
+  return hip_status(t2t::launch_linear(w_transposed != 0, static_cast<const __bf16*>(x), x_stride,
+                                       static_cast<const __bf16*>(w), w_stride,
+                                       static_cast<__bf16*>(y), y_stride, M, N, K,
+                                       static_cast<hipStream_t>(stream)),
+                    "t2t_linear launch");
+}
+
 int64_t t2t_wgrad_workspace(int32_t M, int32_t N, int32_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || M % 128 || N % 128 || K % 64) return 0;
   return (int64_t)t2t::wgrad_splits(M, N, K) * M * N * 4;

@@ -200,6 +200,22 @@ Tensor swiglu_backward(const Tensor& g2, const Tensor& dh, at::IntArrayRef shape
   return dgu;
 }
 
+// ---- linear map of token rows: x W^T, or x W (transposed)
+
+Tensor linear(const Tensor& x, const Tensor& w, bool transposed) {
+  const c10::DeviceGuard guard(x.device());
+  const Tensor x2 = rows_of(x, true), w2 = rows_of(w, true);
+  const int64_t M = x2.size(0), K = x2.size(1), N = w2.size(transposed ? 1 : 0);
+  TORCH_CHECK(w2.size(transposed ? 0 : 1) == K, "weight ", w.sizes(), " does not take rows of ", K);
+  std::vector<int64_t> shape = x.sizes().vec();
+  shape.back() = N;
+  Tensor y = at::empty(shape, x.options());
+  check(t2t_linear(x2.data_ptr(), x2.stride(0), w2.data_ptr(), w2.stride(0), transposed,
+                   y.data_ptr(), N, M, N, K, stream_of(x)),
+        "t2t_linear");
+  return y;
+}
+
 // ---- weight gradient dY^T X
 
 Tensor wgrad(const Tensor& dy, const Tensor& x, at::ScalarType out_dtype) {
@@ -314,6 +330,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         [](const Tensor& g2, const Tensor& dh, const std::vector<int64_t>& shape) {
           return swiglu_backward(g2, dh, shape);
         });
+  m.def("linear", &linear);
   m.def("wgrad", [](const Tensor& dy, const Tensor& x, bool f32) {
     return wgrad(dy, x, f32 ? at::kFloat : at::kBFloat16);
   });

@@ -1,10 +1,11 @@
-"""nn.Linear whose weight gradient runs on the gfx950 split-K kernel
-(``t2t_wgrad``).
+"""nn.Linear on the gfx950 kernels: short products (``t2t_linear``) and the
+split-K weight gradient (``t2t_wgrad``).
 
 The layers' projections (tunalab FlexSelfAttention's qkv / out projections
 and GLU's gate_up / down, called from model/modules/layer.py:33-35) are
-bias-free nn.Linear maps over all T tokens.  Their forward and input
-gradient stay library products (hipBLASLt / rocBLAS through torch); the
+bias-free nn.Linear maps over all T tokens.  Over a short sequence their
+forward and input gradient run on the tiles of ``t2t_linear``; over a long
+one they are library products (hipBLASLt / rocBLAS through torch).  The
 weight gradient dW = dY^T X contracts K = T rows into a small output
 (768 x 768 ... 4096 x 768 at configs[4]), which the library runs on 36-192
 output tiles, a fraction of the 256 CUs.  ``t2t_wgrad`` splits K across
@@ -35,20 +36,52 @@ def wgrad(dy: torch.Tensor, x: torch.Tensor, out_dtype: torch.dtype) -> torch.Te
     return _lib.host().wgrad(dy, x, _OUT_F32[out_dtype])
 
 
+# Products of up to this many multiply-adds run on t2t_linear; the line is
+# where its kernel takes as long as the library call's host side (~23 us;
+# 2048 x 4096 x 768 = 6.4e9: 21 us), beyond which the library's kernels are
+# faster (4096 x 2304 x 768 = 7.2e9: 24 against 19.5 us).
+SHORT_PRODUCT = 6.5e9
+
+
+def short_product(x: torch.Tensor, w: torch.Tensor, transposed: bool) -> bool:
+    """Whether x W^T (x W when ``transposed``) of bf16 rows is t2t_linear's:
+    small, contiguous, rows that 16-byte pieces cover, operands under 2 GiB (a
+    product with very few features could reach that)."""
+    n, k = (w.shape[1], w.shape[0]) if transposed else w.shape
+    rows = x.numel() // max(k, 1)
+    return (x.is_cuda and x.device == w.device and x.dtype == torch.bfloat16
+            and w.dtype == torch.bfloat16 and k > 0 and x.shape[-1] == k and k % 8 == 0
+            and w.shape[1] % 8 == 0 and 0 < rows * n * k <= SHORT_PRODUCT
+            and (rows + 128) * k < 1 << 30 and (w.shape[0] + 128) * w.shape[1] < 1 << 30
+            and x.is_contiguous() and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and not torch.is_autocast_enabled())
+
+
+def product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """F.linear(x, w) of tensors that autograd does not watch."""
+    if short_product(x, w, False):
+        return _lib.host().linear(x, w, False)
+    return F.linear(x, w)
+
+
 class WGradLinearFn(torch.autograd.Function):
-    """y = x W^T (bias-free); dX = dY W by the library, dW by t2t_wgrad."""
+    """y = x W^T (bias-free): y and dX = dY W on t2t_linear for short
+    sequences, by the library for long ones; dW by t2t_wgrad."""
 
     @staticmethod
     def forward(ctx, x, weight):
         ctx.save_for_backward(x, weight)
-        return F.linear(x, weight)
+        return product(x, weight)
 
     @staticmethod
     def backward(ctx, dy):
         x, weight = ctx.saved_tensors
         dx = dw = None
         if ctx.needs_input_grad[0]:
-            dx = (dy.reshape(-1, dy.shape[-1]) @ weight.to(dy.dtype)).view(x.shape)
+            if _lib.unwatched(dy, weight) and short_product(dy, weight, True):
+                dx = _lib.host().linear(dy, weight, True)
+            else:
+                dx = (dy.reshape(-1, dy.shape[-1]) @ weight.to(dy.dtype)).view(x.shape)
         if ctx.needs_input_grad[1]:
             if wgrad_applies(dy, x, weight):
                 dw = wgrad(dy, x, weight.dtype)
@@ -60,13 +93,14 @@ class WGradLinearFn(torch.autograd.Function):
 
 class Linear(nn.Linear):
     """nn.Linear (same parameters and state dict); bias-free bf16 maps on the
-    GPU take their weight gradient from t2t_wgrad."""
+    GPU run as WGradLinearFn does."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # (graphs being compiled keep torch's own linear: the Function's
-        # backward calls the library through ctypes)
+        # backward calls the library through its host module)
         if (self.bias is None and x.is_cuda and x.dtype == torch.bfloat16
-                and self.weight.dtype == torch.bfloat16 and not torch.compiler.is_compiling()
-                and not _lib.unwatched(x, self.weight)):
+                and self.weight.dtype == torch.bfloat16 and not torch.compiler.is_compiling()):
+            if _lib.unwatched(x, self.weight):
+                return product(x, self.weight)
             return WGradLinearFn.apply(x, self.weight)
         return super().forward(x)
