@@ -161,6 +161,12 @@ __device__ __forceinline__ void lds_copy16_m0(uint32_t m0, int voff, u32x4 rsrc)
                :
                : "s"(m0), "v"(voff), "s"(rsrc));
 }
+// ... from a 64-bit address per lane (all lanes' 16 bytes are in bounds).
+__device__ __forceinline__ void lds_copy16_at(uint32_t m0, const void* src) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :
+               : "s"(m0), "v"(src));
+}
 __device__ __forceinline__ void lds_copy4_m0(uint32_t m0, int voff, u32x4 rsrc) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
                :

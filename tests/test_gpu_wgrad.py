@@ -29,6 +29,25 @@ def test_wgrad_against_float32(K, M, N, pad_a, pad_b, out_dtype):
     assert torch.equal(wgrad(dy, x, out_dtype), got)  # fixed summation order
 
 
+# One step, fewer steps than buffers, step counts that the splits share out
+# unevenly, grids that 8 does not divide, a row stride past 32 bits over the
+# rows of a step.  A sum of K products of N(0, 1) is about sqrt(K); K roundings
+# of 6e-8 of that in random directions give 6e-8 K (K = 6464: 4e-4), the
+# largest of an output some five times as much: 1e-4 sqrt(K) (8e-3) holds
+# that and is far below one product lost (about 1).
+@pytest.mark.parametrize("K,M,N,lda", [(64, 128, 128, 128), (128, 128, 256, 256),
+                                       (64 * 101, 384, 128, 384), (64 * 37, 640, 896, 640),
+                                       (192, 128, 128, (1 << 24) + 8)])
+def test_wgrad_uneven_splits_and_wide_rows(K, M, N, lda):
+    g = torch.Generator().manual_seed(K + M)
+    dy = torch.empty(K, lda, dtype=torch.bfloat16, device=DEV)[:, lda - M:]
+    dy.copy_(torch.randn(K, M, generator=g))
+    x = torch.randn(K, N, generator=g).to(torch.bfloat16).to(DEV)
+    got = wgrad(dy, x, torch.float32)
+    ref = dy.double().t() @ x.double()
+    torch.testing.assert_close(got.double(), ref, rtol=0, atol=1e-4 * K ** 0.5)
+
+
 def test_linear_gradients_match_nn_linear():
     torch.manual_seed(0)
     lin = Linear(256, 384, bias=False).to(DEV).to(torch.bfloat16)
