@@ -33,6 +33,8 @@
 // Work-groups are dispatched longest row first (row_order); with grouped-query
 // heads the heads of one KV head and row run back to back on one XCD
 // (head_and_slot), so their K/V copies are served by that XCD's L2.
+#include <type_traits>
+
 #include "attn_kernels.h"
 
 namespace t2t {
@@ -50,29 +52,62 @@ struct FwdParams {
   MaskTables m;
 };
 
+// unit_dma of two consecutive units, the second's rows unit_off bytes on and
+// its last instruction two waves on.
+template <int D, int SK>
+__device__ __forceinline__ void two_units_dma(__bf16* dst, __amdgpu_buffer_rsrc_t src,
+                                              const int* voff, int row_off, int unit_off, int wave,
+                                              int extra_wave) {
+  using U = UnitDma<D, kWaves, SK>;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    __bf16* to = dst + u * U::kElems;
+    const int off = row_off + u * unit_off;
+#pragma unroll
+    for (int j = 0; j < U::kPerWave; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          src, (__attribute__((address_space(3))) void*)(to + (wave + kWaves * j) * 64 * 8), 16,
+          voff[j] + off, 0, 0, 0);
+    if (wave == extra_wave + 2 * u)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          src, (__attribute__((address_space(3))) void*)(to + (U::kInsts - 1) * 64 * 8), 16,
+          voff[U::kPerWave] + off, 0, 0, 0);
+  }
+}
+
 }  // namespace
 
-template <int D, int SK>
+// KP = 1: 128 queries a work-group, SK keys a step.  KP = 2, for short grids
+// (launch_attn_fwd_bf16): 64 queries, 2 SK keys a step shared out between the
+// two waves of each 32 queries, whose sums meet at the end.  A third step in
+// flight, as a ring with counted waits, measured the same (17.9 us at 8 heads
+// x 2048 tokens): a step takes what its MFMA and softmax chain takes, not the
+// copies' latency.
+template <int D, int SK, int KP>
 __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(FwdParams p) {
   constexpr int KS = D / 16;     // MFMA k-steps over the head dim
   constexpr int DT = D / 32;     // 32-wide output column tiles
-  constexpr int NB = SK / 32;    // 32-key blocks per step
-  constexpr int NS = kTile / SK; // steps per KV tile
+  constexpr int NB = SK / 32;    // 32-key blocks per step (and wave)
+  constexpr int NS = kTile / (SK * KP);  // steps per KV tile
   constexpr int PK = SK / 16;    // P V k-steps per step
   using U = UnitDma<D, kWaves, SK>;
-  __shared__ __bf16 k_a[U::kElems], k_b[U::kElems], v_a[U::kElems], v_b[U::kElems];
+  constexpr int kElems = KP * U::kElems;
+  __shared__ __bf16 k_a[kElems], k_b[kElems], v_a[kElems], v_b[kElems];
 
   const int b = blockIdx.z;
   const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = tid & 63;
   const int g = lane >> 5, n = lane & 31;
   const int T = p.T, nt = p.m.nt;
   int h, slot;
-  head_and_slot(p.Hq, p.Hkv, nt, h, slot);
+  head_and_slot(p.Hq, p.Hkv, nt * KP, h, slot);
   const int hk = h / (p.Hq / p.Hkv);
   const int mb = p.m.Bm > 1 ? b : 0;
-  const int qt = uniform(p.m.row_order[(size_t)mb * nt + slot]);
+  const int qt = uniform(p.m.row_order[(size_t)mb * nt + slot / KP]);
   const int q0 = qt * kTile;
-  const int qloc = 32 * wave + n;  // query row within the tile
+  // this wave's 32 queries and (KP = 2) share of a step's keys
+  const int qg = KP == 1 ? wave : wave & 1, kp = KP == 1 ? 0 : wave >> 1;
+  const int qw = kTile / KP * (KP == 1 ? 0 : slot & 1);  // work-group's first row in the tile
+  const int qloc = qw + 32 * qg + n;                     // query row within the tile
   const int qrow = q0 + qloc;
   const bool qvalid = qrow < T;
   const float c = p.scale_log2;
@@ -115,14 +150,19 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(FwdParams p)
   };
   int tiles_v = load_chunk(0);
   auto tile_of = [&](int it) { return __builtin_amdgcn_readlane(tiles_v, it & 63); };
-  // K and V rows [t0, t0 + SK) into one step's units.
+  // K and V rows [t0, t0 + SK KP) into one step's units.
   // (t0 >= T, e.g. past the last tile, copies zeros.)
   const auto krs = slice_rsrc(kbase, p.k_st, T, D);
   const auto vrs = slice_rsrc(vbase, p.v_st, T, D);
   const int k_row2 = (int)p.k_st * 2, v_row2 = (int)p.v_st * 2;
   auto load_step = [&](__bf16* kd, __bf16* vd, int t0) {
-    unit_dma<D, kWaves, SK>(kd, krs, koff, t0 * k_row2, wave, 0);
-    unit_dma<D, kWaves, SK>(vd, vrs, voff, t0 * v_row2, wave, 1);
+    if constexpr (KP == 1) {
+      unit_dma<D, kWaves, SK>(kd, krs, koff, t0 * k_row2, wave, 0);
+      unit_dma<D, kWaves, SK>(vd, vrs, voff, t0 * v_row2, wave, 1);
+    } else {
+      two_units_dma<D, SK>(kd, krs, koff, t0 * k_row2, SK * k_row2, wave, 0);
+      two_units_dma<D, SK>(vd, vrs, voff, t0 * v_row2, SK * v_row2, wave, 1);
+    }
   };
   // The lane's four bitmap words (its query row of the tile's row-major
   // bitmap) of iteration it, loaded into registers one tile ahead.  (Tiles
@@ -147,7 +187,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(FwdParams p)
   // seed), which keeps each contraction one straight-line run of NB
   // interleaved accumulator chains.
   auto step = [&](const __bf16* kt_lds, const __bf16* vt_lds, uint32_t w0, uint32_t w1,
-                  bool partial) {
+                  bool partial) __attribute__((always_inline)) {
     const uint32_t w_any = NB == 2 ? (w0 | w1) : w0, w_all = NB == 2 ? (w0 & w1) : w0;
     if (partial && __ballot(w_any != 0u) == 0ull) return;
     f32x16 st[NB];
@@ -262,28 +302,91 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(FwdParams p)
     if (npart > 0) mb_next = load_bits(0, k0_next / kTile);
     load_step(k_a, v_a, k0_next);
   }
-  for (int it = 0; it < ntiles; ++it) {
-    const bool partial = it < npart;
-    const int k0 = k0_next;
-    const uint4 mbits = partial ? mb_next : make_uint4(~0u, ~0u, ~0u, ~0u);
+  if constexpr (KP == 1) {
+    for (int it = 0; it < ntiles; ++it) {
+      const bool partial = it < npart;
+      const int k0 = k0_next;
+      const uint4 mbits = partial ? mb_next : make_uint4(~0u, ~0u, ~0u, ~0u);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      // Keys [k0 + SK s, + SK): their units (and at s = 0 the tile's bitmap
-      // words) have landed; the other buffer's units are free again.
-      dma_barrier();
-      __bf16 *kc = (s & 1) ? k_b : k_a, *vc = (s & 1) ? v_b : v_a;
-      __bf16 *kn = (s & 1) ? k_a : k_b, *vn = (s & 1) ? v_a : v_b;
-      if (s + 1 < NS) {
-        load_step(kn, vn, k0 + SK * (s + 1));
-      } else if (it + 1 < ntiles) {
-        if (((it + 1) & 63) == 0) tiles_v = load_chunk((it + 1) >> 6);
-        k0_next = tile_of(it + 1) * kTile;
-        if (it + 1 < npart) mb_next = load_bits(it + 1, k0_next / kTile);
-        load_step(kn, vn, k0_next);
+      for (int s = 0; s < NS; ++s) {
+        // Keys [k0 + SK s, + SK): their units (and at s = 0 the tile's bitmap
+        // words) have landed; the other buffer's units are free again.
+        dma_barrier();
+        __bf16 *kc = (s & 1) ? k_b : k_a, *vc = (s & 1) ? v_b : v_a;
+        __bf16 *kn = (s & 1) ? k_a : k_b, *vn = (s & 1) ? v_a : v_b;
+        if (s + 1 < NS) {
+          load_step(kn, vn, k0 + SK * (s + 1));
+        } else if (it + 1 < ntiles) {
+          if (((it + 1) & 63) == 0) tiles_v = load_chunk((it + 1) >> 6);
+          k0_next = tile_of(it + 1) * kTile;
+          if (it + 1 < npart) mb_next = load_bits(it + 1, k0_next / kTile);
+          load_step(kn, vn, k0_next);
+        }
+        auto word = [&](int i) { return i == 0 ? mbits.x : i == 1 ? mbits.y : i == 2 ? mbits.z : mbits.w; };
+        step(kc, vc, word(NB * s), word(NB * s + NB - 1), partial);
       }
-      auto word = [&](int i) { return i == 0 ? mbits.x : i == 1 ? mbits.y : i == 2 ? mbits.z : mbits.w; };
-      step(kc, vc, word(NB * s), word(NB * s + NB - 1), partial);
     }
+  } else {
+    // As above; a tile of one step leaves the next tile the other buffers.
+    auto tile = [&](int it, auto first) __attribute__((always_inline)) {
+      constexpr int F = decltype(first)::value;
+      const bool partial = it < npart;
+      const int k0 = k0_next;
+      const uint4 mbits = partial ? mb_next : make_uint4(~0u, ~0u, ~0u, ~0u);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        dma_barrier();
+        __bf16 *kc = ((s + F) & 1) ? k_b : k_a, *vc = ((s + F) & 1) ? v_b : v_a;
+        __bf16 *kn = ((s + F) & 1) ? k_a : k_b, *vn = ((s + F) & 1) ? v_a : v_b;
+        if (s + 1 < NS) {
+          load_step(kn, vn, k0 + SK * KP * (s + 1));
+        } else if (it + 1 < ntiles) {
+          if (((it + 1) & 63) == 0) tiles_v = load_chunk((it + 1) >> 6);
+          k0_next = tile_of(it + 1) * kTile;
+          if (it + 1 < npart) mb_next = load_bits(it + 1, k0_next / kTile);
+          load_step(kn, vn, k0_next);
+        }
+        auto word = [&](int i) { return i == 0 ? mbits.x : i == 1 ? mbits.y : i == 2 ? mbits.z : mbits.w; };
+        const uint32_t w0 = kp ? word(NB * (KP * s + 1)) : word(NB * KP * s);
+        const uint32_t w1 = kp ? word(NB * (KP * s + 2) - 1) : word(NB * (KP * s + 1) - 1);
+        step(kc + kp * U::kElems, vc + kp * U::kElems, w0, w1, partial);
+      }
+    };
+    if constexpr (NS % 2 == 0) {
+      for (int it = 0; it < ntiles; ++it) tile(it, std::integral_constant<int, 0>{});
+    } else {
+      for (int it = 0; it < ntiles; it += 2) {
+        tile(it, std::integral_constant<int, 0>{});
+        if (it + 1 < ntiles) tile(it + 1, std::integral_constant<int, 1>{});
+      }
+    }
+
+    // The two shares of a query meet in LDS (a copy buffer per pair of waves);
+    // the first wave sums them against their larger reference.
+    static_assert((16 * DT + 2) * 64 * 4 <= kElems * 2, "a wave's sums fit a buffer");
+    __syncthreads();
+    float* share = reinterpret_cast<float*>(qg ? v_a : k_a) + lane;
+    if (kp == 1) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) share[(16 * dt + i) * 64] = oacc[dt][i];
+      share[16 * DT * 64] = m_ref;
+      share[(16 * DT + 1) * 64] = l_run;
+    }
+    __syncthreads();
+    if (kp == 1) return;
+    const float m = share[16 * DT * 64], l = share[(16 * DT + 1) * 64];
+    const float mx = fmaxf(m_ref, m);
+    // (a share without a key has no reference and sums of zero)
+    const float x = m_ref == -INFINITY ? 0.f : fast_exp2((m_ref - mx) * c);
+    const float y = m == -INFINITY ? 0.f : fast_exp2((m - mx) * c);
+    m_ref = mx;
+    l_run = l_run * x + l * y;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) oacc[dt][i] = oacc[dt][i] * x + share[(16 * dt + i) * 64] * y;
   }
 
   if (qvalid) {
@@ -318,14 +421,27 @@ hipError_t launch_attn_fwd_bf16(const TensorView& q, const TensorView& k, const 
   p.scale_log2 = dims.scale * kLog2e;
   p.m = mask;
   if (mask.nt == 0 || dims.B == 0 || dims.Hq == 0) return hipSuccess;
-  dim3 grid(dims.Hq, mask.nt, dims.B);
   // Keys per step: 64 at D = 64 (128 VGPRs, 36 KiB: four work-groups per
   // CU), 32 at D = 128 (158 VGPRs, 36 KiB: three per CU, where 64-key halves
   // hold 180 VGPRs and 68 KiB, two per CU).
+  //
+  // Up to two 128-query work-groups per CU the time is that of the longest
+  // row, one wave's chain of dependent steps: work-groups of 64 queries halve
+  // the chain (72 KiB of LDS: two per CU).  Beyond, K and V being read twice
+  // as often costs more.  us, 128 / 64 queries, rows of linked documents,
+  // D = 64: 8 x 512 (heads x tokens; 32 groups) 13.1 / 10.7, 12 x 2048 (192)
+  // 22.3 / 18.9, 16 x 4096 (512) 43.8 / 34.5, 24 x 4096 (768) 49 / 52;
+  // D = 128: 17.8 / 13.6, 32.7 / 26.3, 64 / 48.5, 73 / 77.
+  const bool split = (int64_t)dims.Hq * mask.nt * dims.B <= 2 * 256;
+  auto launch = [&](auto kernel, int parts) {
+    hipLaunchKernelGGL(kernel, dim3(dims.Hq, mask.nt * parts, dims.B), dim3(kThreads), 0, stream,
+                       p);
+  };
   if (dims.D == 64)
-    hipLaunchKernelGGL((attn_fwd_bf16_kernel<64, 64>), grid, dim3(kThreads), 0, stream, p);
+    split ? launch(attn_fwd_bf16_kernel<64, 64, 2>, 2) : launch(attn_fwd_bf16_kernel<64, 64, 1>, 1);
   else
-    hipLaunchKernelGGL((attn_fwd_bf16_kernel<128, 32>), grid, dim3(kThreads), 0, stream, p);
+    split ? launch(attn_fwd_bf16_kernel<128, 32, 2>, 2)
+          : launch(attn_fwd_bf16_kernel<128, 32, 1>, 1);
   return hipGetLastError();
 }
 

@@ -109,6 +109,37 @@ def test_gqa_group_sizes(B, Hq, Hkv, T, D, gpu_device):
     _oracle_check(rows, B, Hq, Hkv, T, D, seed=Hq + T, device=gpu_device)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [96, 300, 700])
+def test_forward_of_short_and_of_long_grids(T, D, gpu_device):
+    """Up to 512 (head, 128-query tile) pairs the forward runs on 64-query
+    work-groups that share out the keys, beyond on 128-query ones: the same
+    rows on both sides of the line, against the oracle and each other (the
+    probabilities of both are rounded to bf16 against references that may
+    differ, half an ulp each: 2^-8 of the output's scale, and the outputs to
+    bf16: 2^-8 of their own)."""
+    rows = [random_row(T, np.random.default_rng(T), words=1, uncovered=True, max_doc=250)]
+    _oracle_check(rows, 1, 4, 2, T, D, seed=T, device=gpu_device, bwd=False)
+    bm = _mask_from_rows(rows, gpu_device)
+    q, k, v, _ = _inputs(1, 4, 2, T, D, T, gpu_device)
+    copies = 512 // (4 * ((T + 127) // 128))
+
+    def run(n):
+        return flex_attention(*(x.repeat(n, 1, 1, 1) for x in (q, k, v)), block_mask=bm,
+                              enable_gqa=True, return_lse=True)
+
+    short, lse = run(1)
+    for n in (copies, copies + 1):
+        out, out_lse = run(n)
+        assert torch.equal(out, out[:1].expand_as(out))
+        assert torch.equal(out_lse, out_lse[:1].expand_as(out_lse))
+        if n == copies:
+            assert torch.equal(out[:1], short) and torch.equal(out_lse[:1], lse)
+        else:
+            assert_close(out[:1], short, 2 ** -7, 2 ** -7, f"both forms T{T} D{D}")
+            assert_close(out_lse[:1], lse, 1e-4, 1e-4, f"lse of both forms T{T} D{D}")
+
+
 @pytest.mark.parametrize("scale", [0.02, 0.5])
 def test_explicit_scale(scale, gpu_device):
     """A non-default scale reaches the forward's score scaling and the
