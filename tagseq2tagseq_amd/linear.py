@@ -7,7 +7,7 @@ bias-free nn.Linear maps over all T tokens.  Over a short sequence their
 forward and input gradient run on the tiles of ``t2t_linear``; over a long
 one they are library products (hipBLASLt / rocBLAS through torch).  The
 weight gradient dW = dY^T X contracts K = T rows into a small output
-(768 x 768 ... 4096 x 768 at configs[4]), which the library runs on 36-192
+(768 x 768 ... 4096 x 768 over 16384 tokens), which the library runs on 36-192
 output tiles, a fraction of the 256 CUs.  ``t2t_wgrad`` splits K across
 work-groups into fp32 partials and sums them in a fixed order.
 """
