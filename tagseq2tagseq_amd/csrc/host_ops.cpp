@@ -32,6 +32,12 @@ void check(int rc, const char* what) {
   TORCH_CHECK(rc == T2T_OK, what, " failed (status ", rc, "): ", t2t_last_error());
 }
 
+// The kernels get plain addresses: one of host memory would fault the GPU.
+template <typename... Ts>
+void need_gpu(const Ts&... t) {
+  TORCH_CHECK((t.is_cuda() && ...), "the gfx950 kernels need ROCm GPU tensors");
+}
+
 int weight_code(const Tensor& w) {
   TORCH_CHECK(w.scalar_type() == at::kBFloat16 || w.scalar_type() == at::kFloat,
               "weight dtype ", w.scalar_type(), " (bfloat16 or float32)");
@@ -64,6 +70,7 @@ const t2t_block_mask* mask_at(int64_t address) {
 
 std::tuple<Tensor, Tensor> attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v,
                                     int64_t mask, double scale) {
+  need_gpu(q, k, v);
   const c10::DeviceGuard guard(q.device());
   const int64_t B = q.size(0), Hq = q.size(1), T = q.size(2), D = q.size(3), Hkv = k.size(1);
   // [B, T, Hq, D] storage seen as [B, Hq, T, D]: the module's output
@@ -81,6 +88,7 @@ std::tuple<Tensor, Tensor> attn_fwd(const Tensor& q, const Tensor& k, const Tens
 std::tuple<Tensor, Tensor, Tensor> attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v,
                                             const Tensor& out, const Tensor& dout_in,
                                             const Tensor& lse2, int64_t mask, double scale) {
+  need_gpu(q, k, v, out, dout_in, lse2);
   const c10::DeviceGuard guard(q.device());
   const int64_t B = q.size(0), Hq = q.size(1), T = q.size(2), D = q.size(3), Hkv = k.size(1);
   const Tensor dout = dout_in.stride(3) == 1 ? dout_in : dout_in.contiguous();
@@ -100,6 +108,7 @@ std::tuple<Tensor, Tensor, Tensor> attn_bwd(const Tensor& q, const Tensor& k, co
 // ---- RMS normalisation
 
 std::tuple<Tensor, Tensor> rms_norm(const Tensor& x, const Tensor& weight, double eps) {
+  need_gpu(x, weight);
   const c10::DeviceGuard guard(x.device());
   const int64_t C = x.size(-1);
   const Tensor xr = rows_of(x, false), w = weight.contiguous();
@@ -114,6 +123,7 @@ std::tuple<Tensor, Tensor> rms_norm(const Tensor& x, const Tensor& weight, doubl
 
 std::tuple<Tensor, Tensor> rms_norm_backward(const Tensor& dy, const Tensor& x,
                                              const Tensor& weight, const Tensor& rstd) {
+  need_gpu(dy, x, weight, rstd);
   const c10::DeviceGuard guard(x.device());
   const int64_t C = x.size(-1);
   const Tensor xr = rows_of(x, false), dyr = rows_of(dy, false), w = weight.contiguous();
@@ -139,7 +149,7 @@ std::tuple<Tensor, Tensor, Tensor> qkv_rope(const Tensor& qkv_in, const Tensor& 
                     " is not 3 * num_heads * head_dim (num_heads=", heads, ")");
   TORCH_CHECK_NOT_IMPLEMENTED(qkv_in.scalar_type() == at::kBFloat16, "qkv dtype ",
                               qkv_in.scalar_type(), " is not supported (bfloat16 only)");
-  TORCH_CHECK(qkv_in.is_cuda(), "the prologue kernel needs ROCm GPU tensors");
+  need_gpu(qkv_in, cos_in, sin_in);
   const c10::DeviceGuard guard(qkv_in.device());
   const Tensor qkv = qkv_in.stride(2) == 1 ? qkv_in : qkv_in.contiguous();
   const Tensor cos = cos_in.contiguous(), sin = sin_in.contiguous();
@@ -158,6 +168,7 @@ std::tuple<Tensor, Tensor, Tensor> qkv_rope(const Tensor& qkv_in, const Tensor& 
 
 Tensor qkv_rope_backward(const Tensor& dq_in, const Tensor& dk_in, const Tensor& dv_in,
                          const Tensor& cos_in, const Tensor& sin_in, int64_t pos0) {
+  need_gpu(dq_in, dk_in, dv_in, cos_in, sin_in);
   const c10::DeviceGuard guard(dq_in.device());
   const int64_t B = dq_in.size(0), H = dq_in.size(1), T = dq_in.size(2), D = dq_in.size(3);
   const Tensor dq = dq_in.stride(3) == 1 ? dq_in : dq_in.contiguous();
@@ -178,6 +189,7 @@ Tensor qkv_rope_backward(const Tensor& dq_in, const Tensor& dk_in, const Tensor&
 // ---- SwiGLU
 
 std::tuple<Tensor, Tensor> swiglu(const Tensor& gu) {
+  need_gpu(gu);
   const c10::DeviceGuard guard(gu.device());
   const Tensor g2 = rows_of(gu, true);
   const int64_t N = g2.size(0), H = g2.size(1) / 2;
@@ -190,6 +202,7 @@ std::tuple<Tensor, Tensor> swiglu(const Tensor& gu) {
 }
 
 Tensor swiglu_backward(const Tensor& g2, const Tensor& dh, at::IntArrayRef shape) {
+  need_gpu(g2, dh);
   const c10::DeviceGuard guard(g2.device());
   const int64_t N = g2.size(0), H = g2.size(1) / 2;
   const Tensor d2 = rows_of(dh, true);
@@ -203,6 +216,7 @@ Tensor swiglu_backward(const Tensor& g2, const Tensor& dh, at::IntArrayRef shape
 // ---- linear map of token rows: x W^T, or x W (transposed)
 
 Tensor linear(const Tensor& x, const Tensor& w, bool transposed) {
+  need_gpu(x, w);
   const c10::DeviceGuard guard(x.device());
   const Tensor x2 = rows_of(x, true), w2 = rows_of(w, true);
   const int64_t M = x2.size(0), K = x2.size(1), N = w2.size(transposed ? 1 : 0);
@@ -219,6 +233,7 @@ Tensor linear(const Tensor& x, const Tensor& w, bool transposed) {
 // ---- weight gradient dY^T X
 
 Tensor wgrad(const Tensor& dy, const Tensor& x, at::ScalarType out_dtype) {
+  need_gpu(dy, x);
   const c10::DeviceGuard guard(x.device());
   const Tensor d2 = rows_of(dy, true), x2 = rows_of(x, true);
   const int64_t K = d2.size(0), M = d2.size(1), N = x2.size(1);
@@ -239,6 +254,7 @@ Tensor wgrad(const Tensor& dy, const Tensor& x, at::ScalarType out_dtype) {
 // are their own.
 std::vector<Tensor> mask_meta(const Tensor& doc, const Tensor& q_bits, const Tensor& kv_bits,
                               int64_t stream) {
+  need_gpu(doc, q_bits, kv_bits);
   const c10::DeviceGuard guard(doc.device());
   const int64_t Bm = doc.size(0), T = doc.size(1), W = q_bits.size(1);
   const int64_t nt = (T + T2T_TILE - 1) / T2T_TILE;
@@ -290,8 +306,10 @@ std::vector<Tensor> token_inputs(const Tensor& lists, int64_t grants, int64_t co
                                  int64_t links, int64_t B, int64_t T, int64_t words,
                                  int64_t max_spans, int64_t max_grants, bool has_grants,
                                  const std::vector<Tensor>& out) {
+  need_gpu(lists);
   const c10::DeviceGuard guard(lists.device());
   std::vector<Tensor> t = out;
+  for (const Tensor& o : t) need_gpu(o);
   if (t.empty()) {
     t.push_back(at::empty({B, T}, lists.options()));
     if (words > 0)
