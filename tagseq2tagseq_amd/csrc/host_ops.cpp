@@ -44,6 +44,17 @@ int weight_code(const Tensor& w) {
   return w.scalar_type() == at::kFloat ? T2T_DTYPE_F32 : T2T_DTYPE_BF16;
 }
 
+// The attention kernels' code of q's dtype, which k, v and (backward) out and
+// dout share: the kernels read what the code says, whatever the tensors hold.
+template <typename... Ts>
+int attention_code(const Tensor& q, const Ts&... others) {
+  const at::ScalarType t = q.scalar_type();
+  TORCH_CHECK_NOT_IMPLEMENTED(t == at::kBFloat16 || t == at::kFloat, "dtype ", t,
+                              " is not supported (bfloat16 or float32)");
+  TORCH_CHECK_VALUE(((others.scalar_type() == t) && ...), "attention operands differ in dtype");
+  return t == at::kFloat ? T2T_DTYPE_F32 : T2T_DTYPE_BF16;
+}
+
 // [B, H, T, D] with unit stride along D; a dimension of size 1 is never stepped.
 t2t_tensor view4(const Tensor& t) {
   TORCH_CHECK_VALUE(t.dim() == 4, "expected a 4-D [B, H, T, D] tensor, got shape ", t.sizes());
@@ -70,6 +81,7 @@ const t2t_block_mask* mask_at(int64_t address) {
 
 std::tuple<Tensor, Tensor> attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v,
                                     int64_t mask, double scale) {
+  const int dtype = attention_code(q, k, v);
   need_gpu(q, k, v);
   const c10::DeviceGuard guard(q.device());
   const int64_t B = q.size(0), Hq = q.size(1), T = q.size(2), D = q.size(3), Hkv = k.size(1);
@@ -79,8 +91,7 @@ std::tuple<Tensor, Tensor> attn_fwd(const Tensor& q, const Tensor& k, const Tens
   Tensor lse2 = at::empty({B, Hq, T}, q.options().dtype(at::kFloat));
   const t2t_tensor qs = view4(q), ks = view4(k), vs = view4(v), os = view4(out);
   check(t2t_attn_fwd(&qs, &ks, &vs, &os, lse2.data_ptr<float>(), B, Hq, Hkv, T, D,
-                     q.scalar_type() == at::kFloat ? T2T_DTYPE_F32 : T2T_DTYPE_BF16,
-                     static_cast<float>(scale), mask_at(mask), stream_of(q)),
+                     dtype, static_cast<float>(scale), mask_at(mask), stream_of(q)),
         "t2t_attn_fwd");
   return {out, lse2};
 }
@@ -88,6 +99,7 @@ std::tuple<Tensor, Tensor> attn_fwd(const Tensor& q, const Tensor& k, const Tens
 std::tuple<Tensor, Tensor, Tensor> attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v,
                                             const Tensor& out, const Tensor& dout_in,
                                             const Tensor& lse2, int64_t mask, double scale) {
+  const int dtype = attention_code(q, k, v, out, dout_in);
   need_gpu(q, k, v, out, dout_in, lse2);
   const c10::DeviceGuard guard(q.device());
   const int64_t B = q.size(0), Hq = q.size(1), T = q.size(2), D = q.size(3), Hkv = k.size(1);
@@ -98,8 +110,7 @@ std::tuple<Tensor, Tensor, Tensor> attn_bwd(const Tensor& q, const Tensor& k, co
   const t2t_tensor qs = view4(q), ks = view4(k), vs = view4(v), os = view4(out),
                    ds = view4(dout), dqs = view4(dq), dks = view4(dk), dvs = view4(dv);
   check(t2t_attn_bwd(&qs, &ks, &vs, &os, &ds, lse2.data_ptr<float>(), delta.data_ptr<float>(),
-                     &dqs, &dks, &dvs, B, Hq, Hkv, T, D,
-                     q.scalar_type() == at::kFloat ? T2T_DTYPE_F32 : T2T_DTYPE_BF16,
+                     &dqs, &dks, &dvs, B, Hq, Hkv, T, D, dtype,
                      static_cast<float>(scale), mask_at(mask), stream_of(q)),
         "t2t_attn_bwd");
   return {dq, dk, dv};

@@ -43,3 +43,31 @@ def test_host_memory_is_refused(name):
     """A kernel that is handed an address of host memory faults the GPU."""
     with pytest.raises(RuntimeError, match="ROCm GPU tensors"):
         _host_tensor_calls()[name]()
+
+
+@pytest.mark.parametrize("dtypes,error,match", [
+    ((torch.float16,) * 5, NotImplementedError, "dtype Half"),
+    ((torch.uint8,) * 5, NotImplementedError, "dtype Byte"),
+    ((torch.float64,) * 5, NotImplementedError, "dtype Double"),
+    ((torch.bfloat16, torch.float32, torch.bfloat16, torch.bfloat16, torch.bfloat16), ValueError,
+     "differ in dtype"),
+    ((torch.float32, torch.float32, torch.bfloat16, torch.float32, torch.float32), ValueError,
+     "differ in dtype"),
+])
+def test_attention_ops_refuse_other_dtypes(dtypes, error, match):
+    """The custom ops, which no caller validates for: 16-bit floats of another
+    format would be read as bfloat16, narrower types past their end."""
+    q, k, v, out, dout = (torch.zeros(1, 2, 128, 64, dtype=t) for t in dtypes)
+    with pytest.raises(error, match=match):
+        torch.ops.t2t.masked_attention(q, k, v, _tables(), 0.1)
+    with pytest.raises(error, match=match):
+        torch.ops.t2t.masked_attention_backward(q, k, v, out, dout, torch.zeros(1, 2, 128),
+                                                _tables(), 0.1)
+
+
+@pytest.mark.parametrize("which", [3, 4])
+def test_attention_backward_refuses_another_dtype_of_out_or_its_gradient(which):
+    t = [torch.zeros(1, 2, 128, 64, dtype=torch.bfloat16) for _ in range(5)]
+    t[which] = t[which].float()
+    with pytest.raises(ValueError, match="differ in dtype"):
+        torch.ops.t2t.masked_attention_backward(*t, torch.zeros(1, 2, 128), _tables(), 0.1)
