@@ -12,6 +12,7 @@ from typing import List
 
 import torch
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libt2t_attn.so")
@@ -125,11 +126,21 @@ def host():
 
 def unwatched(*tensors) -> bool:
     """True when nothing can be watching a call on these tensors -- no graph
-    to record, no forward-mode level, no function transform -- so that it may
-    go to the kernels without an autograd.Function."""
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+    to record, no forward-mode level, function transform, tracer or dispatch
+    mode, no subclass -- so that it may go to the kernels without an
+    autograd.Function."""
+    return forward_ad._current_level < 0 and host().unwatched(*tensors)
+
+
+def replaces_torch(*tensors) -> bool:
+    """True when a kernel may stand in for a torch function of these tensors
+    unseen: as unwatched (a recorded graph, which its caller is, aside), and
+    no torch function mode overrides torch's functions (a device context, as
+    torch.device or torch.set_default_device makes, only acts on factories)."""
+    n = torch._C._len_torch_function_stack()
+    if n and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n)):
         return False
-    return forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
+    return host().plain(*tensors)
 
 
 def check(rc: int, what: str) -> None:

@@ -13,6 +13,9 @@
 // next.
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
 
 #include <tuple>
@@ -339,6 +342,49 @@ std::vector<Tensor> token_inputs(const Tensor& lists, int64_t grants, int64_t co
   return t;
 }
 
+// ---- what may be watching a call
+
+// Nothing but the caller sees the call, and the tensors are what their
+// addresses say: no tracer, dispatch mode or function transform is active,
+// and every argument is a torch.Tensor or Parameter itself (not a subclass)
+// with plain memory of its own (not batched, nested, sparse or lazily
+// negated).  A kernel called on addresses would be missing from a trace, and
+// its output in it is the empty allocation.
+bool plain_call(PyObject* const* args, Py_ssize_t n, bool recorded_counts) {
+  constexpr c10::DispatchKeySet kIndirect{
+      c10::DispatchKey::Batched,    c10::DispatchKey::FuncTorchBatched,
+      c10::DispatchKey::Python,     c10::DispatchKey::NestedTensor,
+      c10::DispatchKey::Negative,   c10::DispatchKey::Conjugate,
+      c10::DispatchKey::ZeroTensor, c10::DispatchKey::Functionalize};
+  if (torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+      c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+    return false;
+  const bool grad = recorded_counts && c10::GradMode::is_enabled();
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    if (!THPVariable_CheckExact(args[i])) return false;
+    const Tensor& t = THPVariable_Unpack(args[i]);
+    if (t.key_set().has_any(kIndirect) || t.layout() != at::kStrided || !t.has_storage() ||
+        (grad && t.requires_grad()))
+      return false;
+  }
+  return true;
+}
+
+PyObject* plain(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return PyBool_FromLong(plain_call(args, n, false));
+}
+
+PyObject* unwatched(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return PyBool_FromLong(plain_call(args, n, true));
+}
+
+PyMethodDef kPredicates[] = {
+    {"plain", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(plain)), METH_FASTCALL,
+     "plain(*tensors): nothing but the caller sees a call on them"},
+    {"unwatched", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(unwatched)),
+     METH_FASTCALL, "plain(*tensors), and no graph records it"},
+    {nullptr, nullptr, 0, nullptr}};
+
 int64_t current_stream(int64_t device) {
   return reinterpret_cast<int64_t>(
       at::hip::getCurrentHIPStreamMasqueradingAsCUDA(static_cast<c10::DeviceIndex>(device))
@@ -366,4 +412,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mask_meta", &mask_meta);
   m.def("token_inputs", &token_inputs);
   m.def("current_stream", &current_stream);
+  if (PyModule_AddFunctions(m.ptr(), kPredicates) != 0) throw py::error_already_set();
 }

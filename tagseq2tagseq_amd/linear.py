@@ -46,10 +46,13 @@ SHORT_PRODUCT = 6.5e9
 def short_product(x: torch.Tensor, w: torch.Tensor, transposed: bool) -> bool:
     """Whether x W^T (x W when ``transposed``) of bf16 rows is t2t_linear's:
     small, contiguous, rows that 16-byte pieces cover, operands under 2 GiB (a
-    product with very few features could reach that)."""
+    product with very few features could reach that), and not a call that a
+    tracer, a mode or a tensor subclass has to see as torch's own."""
+    if not (x.is_cuda and _lib.replaces_torch(x, w)):
+        return False
     n, k = (w.shape[1], w.shape[0]) if transposed else w.shape
     rows = x.numel() // max(k, 1)
-    return (x.is_cuda and x.device == w.device and x.dtype == torch.bfloat16
+    return (x.device == w.device and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and k > 0 and x.shape[-1] == k and k % 8 == 0
             and w.shape[1] % 8 == 0 and 0 < rows * n * k <= SHORT_PRODUCT
             and (rows + 128) * k < 1 << 30 and (w.shape[0] + 128) * w.shape[1] < 1 << 30

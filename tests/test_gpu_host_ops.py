@@ -1,15 +1,19 @@
 """The calls that go to the kernels without an autograd.Function (nothing to
 record) against the same calls with one: equal bits, and still refused where
-the Function refuses (forward-mode and function transforms); row strides and
-sizes that the C++ wrappers copy or pass on."""
+the Function refuses (forward-mode and function transforms) and still seen by
+tracers, modes and subclasses; row strides and sizes that the C++ wrappers copy
+or pass on."""
 import pytest
 import torch
 import torch.autograd.forward_ad as fwad
+from torch._subclasses.fake_tensor import FakeTensor, FakeTensorMode
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.utils.flop_counter import FlopCounterMode
 
 from tagseq2tagseq_amd import _lib, synth
 from tagseq2tagseq_amd.attention import flex_attention
 from tagseq2tagseq_amd.glu import swiglu
-from tagseq2tagseq_amd.linear import Linear
+from tagseq2tagseq_amd.linear import Linear, short_product
 from tagseq2tagseq_amd.mask_creators import create_doc_causal_block_mask
 from tagseq2tagseq_amd.norm import rms_norm
 from tagseq2tagseq_amd.rope import qkv_rope, rope_tables
@@ -64,6 +68,69 @@ def test_unrecorded_calls(name):
             call(dual)
     with torch.no_grad(), pytest.raises(RuntimeError):
         torch.func.vmap(call)(torch.stack([x, x]))
+
+
+@pytest.mark.parametrize("name", [
+    "norm", "norm rows of a wider tensor", "rope", "swiglu", "swiglu of transposed rows",
+    "attention", "attention of [B, T, H, D] storage"])
+def test_traced_calls_run_again(name):
+    """A trace holds the call itself, not the memory that its kernel filled."""
+    x, call = _calls()[name]
+    other = torch.randn_like(x)
+    with torch.no_grad():
+        traced = torch.jit.trace(call, x, check_trace=False)
+        assert torch.equal(traced(other), call(other))
+        assert torch.equal(traced(x), call(x))
+
+
+def _short_linear():
+    lin = Linear(128, 256, bias=False).to(DEV, torch.bfloat16)
+    x = torch.randn(160, 128, device=DEV).to(torch.bfloat16)
+    assert short_product(x, lin.weight, False)
+    return lin, x
+
+
+def test_linear_is_seen_by_tracers_modes_and_subclasses():
+    lin, x = _short_linear()
+    other = torch.randn_like(x)
+    with torch.no_grad():
+        want = torch.nn.functional.linear(other, lin.weight)
+        assert torch.equal(torch.jit.trace(lin, x, check_trace=False)(other), want)
+        graph = make_fx(lin)(x)
+        assert torch.equal(graph(other), want)
+        with FlopCounterMode(display=False) as flops:
+            lin(x)
+        assert flops.get_total_flops() == 2 * 160 * 128 * 256
+        with FakeTensorMode(allow_non_fake_inputs=True) as fake:
+            y = lin(fake.from_tensor(x))
+        assert isinstance(y, FakeTensor) and y.shape == (160, 256)
+
+        class Tagged(torch.Tensor):
+            pass
+
+        assert type(lin(x.as_subclass(Tagged))) is Tagged
+
+        calls = []
+
+        class Seen(torch.overrides.TorchFunctionMode):
+            def __torch_function__(self, func, types, args=(), kwargs=None):
+                calls.append(func)
+                return func(*args, **(kwargs or {}))
+
+        with Seen():
+            assert torch.equal(lin(other), want)
+        assert torch.nn.functional.linear in calls
+
+
+def test_linear_batched_input_gradients():
+    """Batched gradients of a frozen weight's map, as a Jacobian takes them."""
+    lin, x = _short_linear()
+    lin.weight.requires_grad_(False)
+    x = x[:2].requires_grad_(True)
+    dy = torch.randn(3, 2, 256, device=DEV).to(torch.bfloat16)
+    got, = torch.autograd.grad(lin(x), x, dy, is_grads_batched=True)
+    want = dy.float() @ lin.weight.float()
+    torch.testing.assert_close(got.float(), want, rtol=2.0 ** -8, atol=1e-4)
 
 
 def test_library_errors_carry_their_message():

@@ -1,7 +1,12 @@
 """The C++ host side of the per-layer calls: what it refuses before it reaches
-a kernel.  None of these calls gets as far as a launch."""
+a kernel, and when it may be called at all.  No call gets as far as a launch."""
 import pytest
 import torch
+import torch.autograd.forward_ad as fwad
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.utils._python_dispatch import TorchDispatchMode
+from torch.utils.flop_counter import FlopCounterMode
 
 from tagseq2tagseq_amd import _lib, attention, norm, rope  # noqa: F401  (registers the ops)
 from tagseq2tagseq_amd.mask_creators import TokenLists
@@ -71,3 +76,88 @@ def test_attention_backward_refuses_another_dtype_of_out_or_its_gradient(which):
     t[which] = t[which].float()
     with pytest.raises(ValueError, match="differ in dtype"):
         torch.ops.t2t.masked_attention_backward(*t, torch.zeros(1, 2, 128), _tables(), 0.1)
+
+
+class _Plain(torch.Tensor):
+    """A subclass without any behaviour of its own."""
+
+
+class _Through(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+class _Seen(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def _answers(x):
+    return _lib.unwatched(x), _lib.host().plain(x)
+
+
+def test_plain_calls_are_unwatched():
+    x = torch.zeros(2, 8)
+    w = torch.nn.Parameter(x.clone())
+    assert _answers(x) == (True, True) and _answers(w) == (False, True)
+    with torch.no_grad():
+        assert _lib.unwatched(x, w, x.t(), x[1:]) and _lib.replaces_torch(x, w)
+        with torch.device("cpu"):
+            assert _lib.replaces_torch(x, w)
+        with _Seen():
+            assert not _lib.replaces_torch(x, w)
+    with torch.inference_mode():
+        assert _lib.unwatched(torch.zeros(2))
+
+
+@torch.no_grad()
+def test_tracers_modes_and_transforms_watch():
+    x = torch.zeros(2, 8)
+    got = {}
+
+    def look(name):
+        def f(t):
+            got[name] = _answers(t)
+            return t * 2
+        return f
+
+    torch.jit.trace(look("jit"), x, check_trace=False)
+    make_fx(look("make_fx"))(x)
+    make_fx(look("make_fx fake"), tracing_mode="fake")(x)
+    torch.func.vmap(look("vmap"))(x)
+    torch.func.functionalize(look("functionalize"))(x)
+    with FakeTensorMode(allow_non_fake_inputs=True) as fake:
+        look("fake mode")(x)
+    look("fake tensor")(fake.from_tensor(x))
+    for name, mode in (("flops", FlopCounterMode(display=False)), ("mode", _Through())):
+        with mode:
+            look(name)(x)
+    look("subclass")(x.as_subclass(_Plain))
+    look("lazily negated")(torch._neg_view(x))
+    look("sparse")(x.to_sparse())
+    look("sparse rows")(x.to_sparse_csr())
+    look("nested")(torch.nested.nested_tensor([x[0], x[1, :3]]))
+    assert len(got) == 14
+    assert not {n: a for n, a in got.items() if a != (False, False)}
+    with fwad.dual_level():
+        assert not _lib.unwatched(x)
+
+
+def test_batched_gradients_watch():
+    """torch.autograd.grad(is_grads_batched=True) hands a backward batched
+    tensors without a function transform around it."""
+    seen = []
+
+    class Double(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x * 2
+
+        @staticmethod
+        def backward(ctx, dy):
+            seen.append(_answers(dy))
+            return dy * 2
+
+    x = torch.zeros(3, requires_grad=True)
+    torch.autograd.grad(Double.apply(x), x, torch.eye(3), is_grads_batched=True)
+    assert seen == [(False, False)]
