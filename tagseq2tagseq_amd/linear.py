@@ -45,7 +45,7 @@ SHORT_PRODUCT = 6.5e9
 
 def short_product(x: torch.Tensor, w: torch.Tensor, transposed: bool) -> bool:
     """Whether x W^T (x W when ``transposed``) of bf16 rows is t2t_linear's:
-    small, contiguous, rows that 16-byte pieces cover, operands under 2 GiB (a
+    small, contiguous, rows that aligned 16-byte pieces cover, operands under 2 GiB (a
     product with very few features could reach that), and not a call that a
     tracer, a mode or a tensor subclass has to see as torch's own."""
     if not (x.is_cuda and _lib.replaces_torch(x, w)):
@@ -56,7 +56,8 @@ def short_product(x: torch.Tensor, w: torch.Tensor, transposed: bool) -> bool:
             and w.dtype == torch.bfloat16 and k > 0 and x.shape[-1] == k and k % 8 == 0
             and w.shape[1] % 8 == 0 and 0 < rows * n * k <= SHORT_PRODUCT
             and (rows + 128) * k < 1 << 30 and (w.shape[0] + 128) * w.shape[1] < 1 << 30
-            and x.is_contiguous() and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and x.is_contiguous() and w.is_contiguous()
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and not torch.is_autocast_enabled())
 
 

@@ -78,3 +78,33 @@ def test_linear_module_routes(rows, din, dout):
     assert short_product(dy, lin.weight, True) == (din % 8 == 0 and dout % 8 == 0)
     big = int(SHORT_PRODUCT) // (din * dout) + 1
     assert not short_product(x.detach()[:1, :1].expand(1, big, din), lin.weight, False)
+
+
+def _off_by_one(*shape):
+    """Contiguous N(0, 1) rows that start one element past a 16-byte boundary."""
+    n = 1
+    for d in shape:
+        n *= d
+    buf = torch.randn(n + 8, device=DEV).to(torch.bfloat16)
+    t = buf[1:1 + n].view(*shape)
+    assert t.is_contiguous() and t.data_ptr() % 16 == 2
+    return t
+
+
+@pytest.mark.parametrize("din,dout", [(136, 72), (64, 200)])
+def test_linear_of_rows_off_a_16_byte_boundary(din, dout):
+    """Input rows and an incoming gradient that the kernel cannot read in whole
+    pieces: torch's products, as for any other such operand."""
+    lin = Linear(din, dout, bias=False).to(DEV, torch.bfloat16)
+    x, dy = _off_by_one(40, din), _off_by_one(40, dout)
+    want = F.linear(x.float(), lin.weight.float())
+    with torch.no_grad():
+        torch.testing.assert_close(lin(x).float(), want, rtol=2.0 ** -8, atol=1e-4)
+    x = x.requires_grad_(True)
+    y = lin(x)
+    torch.testing.assert_close(y.float(), want, rtol=2.0 ** -8, atol=1e-4)
+    y.backward(dy)
+    torch.testing.assert_close(x.grad.float(), dy.float() @ lin.weight.float(), rtol=2.0 ** -8,
+                               atol=1e-4)
+    torch.testing.assert_close(lin.weight.grad.float(), dy.float().t() @ x.detach().float(),
+                               rtol=2.0 ** -8, atol=1e-4)
