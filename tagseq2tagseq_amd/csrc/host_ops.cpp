@@ -67,13 +67,14 @@ t2t_tensor view4(const Tensor& t) {
 }
 
 // The rows [N, C] of t's last dimension as the kernels read them: unit column
-// stride, row stride a multiple of 8 elements and, where `aligned`, a 16-byte
-// aligned start; anything else is copied.
-Tensor rows_of(const Tensor& t, bool aligned) {
+// stride, row stride a multiple of 8 elements and a 16-byte aligned start;
+// anything else is copied (rows that are contiguous but start between two such
+// boundaries too, which contiguous() would hand back).
+Tensor rows_of(const Tensor& t) {
   Tensor r = t.dim() == 2 ? t : t.reshape({-1, t.size(-1)});
   const bool ok = r.stride(1) == 1 && r.stride(0) % 8 == 0 &&
-                  (!aligned || reinterpret_cast<uintptr_t>(r.data_ptr()) % 16 == 0);
-  return ok ? r : r.contiguous();
+                  reinterpret_cast<uintptr_t>(r.data_ptr()) % 16 == 0;
+  return ok ? r : r.clone(at::MemoryFormat::Contiguous);
 }
 
 const t2t_block_mask* mask_at(int64_t address) {
@@ -125,7 +126,7 @@ std::tuple<Tensor, Tensor> rms_norm(const Tensor& x, const Tensor& weight, doubl
   need_gpu(x, weight);
   const c10::DeviceGuard guard(x.device());
   const int64_t C = x.size(-1);
-  const Tensor xr = rows_of(x, false), w = weight.contiguous();
+  const Tensor xr = rows_of(x), w = weight.contiguous();
   const int64_t N = xr.size(0);
   Tensor y = at::empty(x.sizes(), x.options());
   Tensor rstd = at::empty({N}, x.options().dtype(at::kFloat));
@@ -140,7 +141,7 @@ std::tuple<Tensor, Tensor> rms_norm_backward(const Tensor& dy, const Tensor& x,
   need_gpu(dy, x, weight, rstd);
   const c10::DeviceGuard guard(x.device());
   const int64_t C = x.size(-1);
-  const Tensor xr = rows_of(x, false), dyr = rows_of(dy, false), w = weight.contiguous();
+  const Tensor xr = rows_of(x), dyr = rows_of(dy), w = weight.contiguous();
   const int64_t N = xr.size(0);
   Tensor dx = at::empty(x.sizes(), x.options());
   Tensor dw = at::empty(w.sizes(), w.options());
@@ -205,7 +206,7 @@ Tensor qkv_rope_backward(const Tensor& dq_in, const Tensor& dk_in, const Tensor&
 std::tuple<Tensor, Tensor> swiglu(const Tensor& gu) {
   need_gpu(gu);
   const c10::DeviceGuard guard(gu.device());
-  const Tensor g2 = rows_of(gu, true);
+  const Tensor g2 = rows_of(gu);
   const int64_t N = g2.size(0), H = g2.size(1) / 2;
   std::vector<int64_t> shape = gu.sizes().vec();
   shape.back() = H;
@@ -219,7 +220,7 @@ Tensor swiglu_backward(const Tensor& g2, const Tensor& dh, at::IntArrayRef shape
   need_gpu(g2, dh);
   const c10::DeviceGuard guard(g2.device());
   const int64_t N = g2.size(0), H = g2.size(1) / 2;
-  const Tensor d2 = rows_of(dh, true);
+  const Tensor d2 = rows_of(dh);
   Tensor dgu = at::empty(shape, g2.options());
   check(t2t_swiglu_backward(g2.data_ptr(), g2.stride(0), d2.data_ptr(), d2.stride(0),
                             dgu.data_ptr(), 2 * H, N, H, stream_of(g2)),
@@ -232,7 +233,7 @@ Tensor swiglu_backward(const Tensor& g2, const Tensor& dh, at::IntArrayRef shape
 Tensor linear(const Tensor& x, const Tensor& w, bool transposed) {
   need_gpu(x, w);
   const c10::DeviceGuard guard(x.device());
-  const Tensor x2 = rows_of(x, true), w2 = rows_of(w, true);
+  const Tensor x2 = rows_of(x), w2 = rows_of(w);
   const int64_t M = x2.size(0), K = x2.size(1), N = w2.size(transposed ? 1 : 0);
   TORCH_CHECK(w2.size(transposed ? 0 : 1) == K, "weight ", w.sizes(), " does not take rows of ", K);
   std::vector<int64_t> shape = x.sizes().vec();
@@ -249,7 +250,7 @@ Tensor linear(const Tensor& x, const Tensor& w, bool transposed) {
 Tensor wgrad(const Tensor& dy, const Tensor& x, at::ScalarType out_dtype) {
   need_gpu(dy, x);
   const c10::DeviceGuard guard(x.device());
-  const Tensor d2 = rows_of(dy, true), x2 = rows_of(x, true);
+  const Tensor d2 = rows_of(dy), x2 = rows_of(x);
   const int64_t K = d2.size(0), M = d2.size(1), N = x2.size(1);
   Tensor ws = at::empty({t2t_wgrad_workspace(M, N, K)}, x.options().dtype(at::kByte));
   Tensor out = at::empty({M, N}, x.options().dtype(out_dtype));

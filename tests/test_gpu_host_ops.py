@@ -3,6 +3,8 @@ record) against the same calls with one: equal bits, and still refused where
 the Function refuses (forward-mode and function transforms) and still seen by
 tracers, modes and subclasses; row strides and sizes that the C++ wrappers copy
 or pass on."""
+import math
+
 import pytest
 import torch
 import torch.autograd.forward_ad as fwad
@@ -131,6 +133,43 @@ def test_linear_batched_input_gradients():
     got, = torch.autograd.grad(lin(x), x, dy, is_grads_batched=True)
     want = dy.float() @ lin.weight.float()
     torch.testing.assert_close(got.float(), want, rtol=2.0 ** -8, atol=1e-4)
+
+
+def _off_by_one(*shape):
+    """Contiguous N(0, 1) rows that start one element past a 16-byte boundary."""
+    buf = torch.randn(math.prod(shape) + 8, device=DEV).to(torch.bfloat16)
+    t = buf[1:1 + math.prod(shape)].view(*shape)
+    assert t.is_contiguous() and t.data_ptr() % 16 == 2
+    return t
+
+
+def test_rows_off_a_16_byte_boundary_are_copied():
+    """The kernels read rows in 16-byte pieces, and contiguous() of rows that
+    are contiguous already is no copy."""
+    x, dy = _off_by_one(3, 64, 256), _off_by_one(3, 64, 128)
+    even = x.clone().requires_grad_(True)
+    odd = x.requires_grad_(True)
+    want, got = swiglu(even), swiglu(odd)
+    assert torch.equal(want, got)
+    want.backward(dy.clone())
+    got.backward(dy)
+    assert torch.equal(even.grad, odd.grad)
+    x, host = x.detach(), _lib.host()
+    norm_w = torch.randn(256, device=DEV).to(torch.bfloat16)
+    assert torch.equal(rms_norm(x, norm_w, 1e-6), rms_norm(x.clone(), norm_w, 1e-6))
+    assert torch.equal(host.wgrad(dy, x, True), host.wgrad(dy.clone(), x.clone(), True))
+    w = _off_by_one(128, 256)
+    assert torch.equal(host.linear(x, w, False), host.linear(x.clone(), w.clone(), False))
+    assert torch.equal(host.linear(dy, w, True), host.linear(dy.clone(), w.clone(), True))
+
+
+def test_linear_trains_on_rows_off_a_16_byte_boundary():
+    """Widths whose weight gradient is the split kernel's."""
+    lin = Linear(256, 128, bias=False).to(DEV, torch.bfloat16)
+    x, dy = _off_by_one(128, 256), _off_by_one(128, 128)
+    lin(x.requires_grad_(True)).backward(dy)
+    torch.testing.assert_close(lin.weight.grad.float(), dy.float().t() @ x.detach().float(),
+                               rtol=2.0 ** -8, atol=1e-3)
 
 
 def test_library_errors_carry_their_message():
