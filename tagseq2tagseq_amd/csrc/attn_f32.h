@@ -242,15 +242,20 @@ struct BlockWalk {
   }
 
   // Block i of the chunk: its first token, whether it has both allowed and
-  // masked pairs (mixed), and this lane's mask word (requested for every
-  // block: a conditional load would have to be waited for where its two paths
-  // meet; words of a block that is not mixed are not used).
+  // masked pairs (mixed), and this lane's mask word.  The load is issued for
+  // every block (a conditional one would have to be waited for where its two
+  // paths meet), but through a buffer of no size when the block is not mixed:
+  // a full tile has no slot, and a row without partial tiles need not have a
+  // valid kv_bits_off.
   __device__ __forceinline__ void block(int i, int& base, uint32_t& w, bool& mixed) const {
     const int e = __builtin_amdgcn_readlane(ent, i);
     const int s = __builtin_amdgcn_readlane(slot, i);
     base = 32 * (e & 0x7fffffff);
     mixed = e < 0;
-    w = (words + ((size_t)(uint32_t)s * kTileBitsWords + (e & 3)))[woff];
+    const auto bits = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t*>(words + ((size_t)(uint32_t)s * kTileBitsWords + (e & 3))), 0,
+        mixed ? 4 * (kTileBitsWords - 3) : 0, 0x00020000);
+    w = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(bits, 4 * (int)woff, 0, 0);
   }
 };
 
