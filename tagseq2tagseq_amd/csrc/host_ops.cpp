@@ -395,23 +395,26 @@ int64_t current_stream(int64_t device) {
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.def("attn_fwd", &attn_fwd);
-  m.def("attn_bwd", &attn_bwd);
-  m.def("rms_norm", &rms_norm);
-  m.def("rms_norm_backward", &rms_norm_backward);
-  m.def("qkv_rope", &qkv_rope);
-  m.def("qkv_rope_backward", &qkv_rope_backward);
-  m.def("swiglu", &swiglu);
+  // a launch may wait on a full queue, an allocation on the device: other
+  // Python threads run meanwhile
+  const auto no_gil = py::call_guard<py::gil_scoped_release>();
+  m.def("attn_fwd", &attn_fwd, no_gil);
+  m.def("attn_bwd", &attn_bwd, no_gil);
+  m.def("rms_norm", &rms_norm, no_gil);
+  m.def("rms_norm_backward", &rms_norm_backward, no_gil);
+  m.def("qkv_rope", &qkv_rope, no_gil);
+  m.def("qkv_rope_backward", &qkv_rope_backward, no_gil);
+  m.def("swiglu", &swiglu, no_gil);
   m.def("swiglu_backward",
         [](const Tensor& g2, const Tensor& dh, const std::vector<int64_t>& shape) {
           return swiglu_backward(g2, dh, shape);
-        });
-  m.def("linear", &linear);
+        }, no_gil);
+  m.def("linear", &linear, no_gil);
   m.def("wgrad", [](const Tensor& dy, const Tensor& x, bool f32) {
     return wgrad(dy, x, f32 ? at::kFloat : at::kBFloat16);
-  });
-  m.def("mask_meta", &mask_meta);
-  m.def("token_inputs", &token_inputs);
+  }, no_gil);
+  m.def("mask_meta", &mask_meta, no_gil);
+  m.def("token_inputs", &token_inputs, no_gil);
   m.def("current_stream", &current_stream);
   if (PyModule_AddFunctions(m.ptr(), kPredicates) != 0) throw py::error_already_set();
 }

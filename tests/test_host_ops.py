@@ -1,5 +1,9 @@
 """The C++ host side of the per-layer calls: what it refuses before it reaches
 a kernel, and when it may be called at all.  No call gets as far as a launch."""
+import sys
+import threading
+import time
+
 import pytest
 import torch
 import torch.autograd.forward_ad as fwad
@@ -161,3 +165,33 @@ def test_batched_gradients_watch():
     x = torch.zeros(3, requires_grad=True)
     torch.autograd.grad(Double.apply(x), x, torch.eye(3), is_grads_batched=True)
     assert seen == [(False, False)]
+
+
+def test_host_calls_release_the_gil():
+    """Another Python thread runs while a call of the host module is under way
+    (a launch that waits on a full queue would stop it otherwise).  The switch
+    interval keeps the interpreter itself from handing the GIL over."""
+    x, host = torch.zeros(4, 128, dtype=torch.bfloat16), _lib.host()
+    go, ran = threading.Lock(), []
+    go.acquire()
+
+    def other():
+        with go:
+            ran.append(True)
+
+    before = sys.getswitchinterval()
+    thread = threading.Thread(target=other)
+    thread.start()
+    try:
+        sys.setswitchinterval(1000.0)
+        end = time.perf_counter() + 5.0
+        go.release()
+        while not ran and time.perf_counter() < end:
+            try:
+                host.swiglu(x)  # refused: host memory
+            except RuntimeError:
+                pass
+        assert ran
+    finally:
+        sys.setswitchinterval(before)
+        thread.join()
