@@ -160,6 +160,7 @@ std::tuple<Tensor, Tensor> rms_norm_backward(const Tensor& dy, const Tensor& x,
 std::tuple<Tensor, Tensor, Tensor> qkv_rope(const Tensor& qkv_in, const Tensor& cos_in,
                                             const Tensor& sin_in, int64_t heads, int64_t pos0) {
   TORCH_CHECK_VALUE(qkv_in.dim() == 3, "qkv must be [B, T, 3 C], got shape ", qkv_in.sizes());
+  TORCH_CHECK_VALUE(heads > 0, "num_heads=", heads, " must be positive");
   TORCH_CHECK_VALUE(qkv_in.size(2) % (3 * heads) == 0, "last dim ", qkv_in.size(2),
                     " is not 3 * num_heads * head_dim (num_heads=", heads, ")");
   TORCH_CHECK_NOT_IMPLEMENTED(qkv_in.scalar_type() == at::kBFloat16, "qkv dtype ",

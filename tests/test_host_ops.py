@@ -1,5 +1,7 @@
 """The C++ host side of the per-layer calls: what it refuses before it reaches
 a kernel, and when it may be called at all.  No call gets as far as a launch."""
+import os
+import subprocess
 import sys
 import threading
 import time
@@ -195,3 +197,18 @@ def test_host_calls_release_the_gil():
     finally:
         sys.setswitchinterval(before)
         thread.join()
+
+
+@pytest.mark.parametrize("heads", [0, -2])
+def test_rope_refuses_a_head_count_that_is_not_positive(heads):
+    """An integer division by zero would end the process."""
+    code = ("import torch, tagseq2tagseq_amd.rope as r\n"
+            "t = torch.zeros(8, 32)\n"
+            "try:\n"
+            f"    r.qkv_rope(torch.zeros(1, 8, 384, dtype=torch.bfloat16), t, t, {heads})\n"
+            "except ValueError as e:\n"
+            "    assert 'num_heads' in str(e), e\n"
+            "    print('refused')\n")
+    got = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True,
+                         cwd=os.path.dirname(_lib.HERE))
+    assert got.stdout == "refused\n", (got.returncode, got.stderr[-500:])
