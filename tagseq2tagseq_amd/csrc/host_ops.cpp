@@ -322,6 +322,8 @@ std::vector<Tensor> token_inputs(const Tensor& lists, int64_t grants, int64_t co
                                  int64_t links, int64_t B, int64_t T, int64_t words,
                                  int64_t max_spans, int64_t max_grants, bool has_grants,
                                  const std::vector<Tensor>& out) {
+  TORCH_CHECK(out.empty() || words == 0 || out.size() == 3,
+              "doc, q_bits and kv_bits are needed to overwrite ", words, " words a token");
   need_gpu(lists);
   const c10::DeviceGuard guard(lists.device());
   std::vector<Tensor> t = out;

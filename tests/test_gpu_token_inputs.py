@@ -113,3 +113,16 @@ def test_creators_end_to_end():
     ref2 = mo.block_mask_tables(mo.document_ids(2048, row.spans))
     assert np.array_equal(bm2.kv_num_blocks[0, 0].cpu().numpy(), ref2["kv_num_blocks"])
     assert np.array_equal(bm2.full_kv_num_blocks[0, 0].cpu().numpy(), ref2["full_kv_num_blocks"])
+
+
+def test_build_returns_what_it_overwrites():
+    """Of lists without words too, whose words are left alone."""
+    spans = [[synth.DocSpan(3, 0, 100)]]
+    linked = TokenLists(128, spans, DEV, words=1, link_rows=[np.ones((1, 1), dtype=np.uint64)])
+    out = linked.build()
+    kept = [t.clone() for t in out]
+    out[0].zero_()
+    for lists in (linked, TokenLists(128, spans, DEV)):
+        got = lists.build(out)
+        assert all(a is b for a, b in zip(got, out)) and len(got) == 3
+        assert all(torch.equal(a, b) for a, b in zip(out, kept))

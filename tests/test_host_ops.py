@@ -6,6 +6,7 @@ import sys
 import threading
 import time
 
+import numpy as np
 import pytest
 import torch
 import torch.autograd.forward_ad as fwad
@@ -212,3 +213,10 @@ def test_rope_refuses_a_head_count_that_is_not_positive(heads):
     got = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True,
                          cwd=os.path.dirname(_lib.HERE))
     assert got.stdout == "refused\n", (got.returncode, got.stderr[-500:])
+
+
+def test_overwriting_token_inputs_needs_the_words_too():
+    lists = TokenLists(128, [[DocSpan(0, 0, 128)]], torch.device("cpu"), words=1,
+                       link_rows=[np.ones((1, 1), dtype=np.uint64)])
+    with pytest.raises(RuntimeError, match="q_bits and kv_bits are needed"):
+        lists.build((torch.zeros(1, 128, dtype=torch.int32), None, None))
