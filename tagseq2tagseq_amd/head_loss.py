@@ -60,7 +60,8 @@ def _head_pass(x, weight, targets, ignore_index: int, chunk: Optional[int], grad
         raise ValueError(f"{t.numel()} targets for {N} rows")
     if weight.shape[1] != D:
         raise ValueError(f"weight {tuple(weight.shape)} does not match rows of width {D}")
-    if ld == V and weight.dtype == torch.bfloat16 and weight.is_contiguous():
+    if (ld == V and weight.device == dev and weight.dtype == torch.bfloat16
+            and weight.is_contiguous()):
         w = weight.detach()
     else:
         w = torch.empty((ld, D), dtype=torch.bfloat16, device=dev)

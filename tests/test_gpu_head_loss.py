@@ -11,7 +11,7 @@ import torch
 import torch.nn.functional as F
 
 from tagseq2tagseq_amd import _lib
-from tagseq2tagseq_amd.head_loss import head_cross_entropy
+from tagseq2tagseq_amd.head_loss import head_cross_entropy, head_loss_value
 from tagseq2tagseq_amd.modules import LinearCELoss
 
 pytestmark = pytest.mark.gpu
@@ -221,3 +221,14 @@ def test_head_loss_takes_host_targets_and_checks_shapes():
         head_cross_entropy(x, w, t[:15])
     with pytest.raises(ValueError):
         head_cross_entropy(x, torch.randn(40, 32, device=DEV), t)
+
+
+@pytest.mark.parametrize("V", [64, 61])
+def test_head_loss_of_a_weight_on_another_device(V):
+    """The weight is copied to the rows' device, whether or not its vocabulary
+    needs padding."""
+    g = torch.Generator(device=DEV).manual_seed(V)
+    x = torch.randn(40, 32, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.randn(V, 32, generator=g, device=DEV).to(torch.bfloat16)
+    t = torch.randint(0, V, (40,), generator=g, device=DEV)
+    assert torch.equal(head_loss_value(x, w.cpu(), t), head_loss_value(x, w, t))
