@@ -214,7 +214,7 @@ def profile_mfma(masks: str, seed: int, out_path: str) -> None:
     lines = ["# MFMA-busy fraction of the attention kernels per bench_layer point (MI355X, bf16):",
              "# SQ_VALU_MFMA_BUSY_CYCLES summed over a kernel's dispatches / (1024 SIMDs x 2.4 GHz x",
              f"# their summed durations), {PASS_CALLS} layer fwd+bwd calls per point after the mask build.",
-             "# command (repo root, GPU box):",
+             "# command (repo root):",
              f"#   python -m tagseq2tagseq_amd.bench_layer --masks {masks} --seed {seed} "
              f"--profile-mfma {os.path.relpath(out_path, ROOT)}",
              ""]

@@ -40,6 +40,13 @@ def wgrad(dy: torch.Tensor, x: torch.Tensor, out_dtype: torch.dtype) -> torch.Te
 # where its kernel takes as long as the library call's host side (~23 us;
 # 2048 x 4096 x 768 = 6.4e9: 21 us), beyond which the library's kernels are
 # faster (4096 x 2304 x 768 = 7.2e9: 24 against 19.5 us).
+# Where nothing waits for the host (a captured graph, a full queue) only the
+# kernels count: the input gradient's is 0 to 55 % faster than the library's
+# up to here, with few exceptions (6144 x 768 x 768 14.2 against 13.4 us, 2048
+# x 3072 x 1024 28.7 / 24.5), the forward's 5 to 40 % faster up to about 2.5e9
+# (512 x 4096 x 1024 11.8 / 9.7) and up to 23 % slower from 3e9 on (3072 x
+# 2304 x 768 20.7 / 15.9, 2048 x 4096 x 768 19.1 / 17.4).  The line does not
+# move with that: a replayed graph has the bits of the eager call.
 SHORT_PRODUCT = 6.5e9
 
 

@@ -111,7 +111,7 @@ def trace(kt_dir: str, bench_json: str, cfg: str, bench_args: str = "") -> str:
     lines = [
         f"# rocprofv3 kernel trace -- {_label(cfg)} ({WORKLOADS.get(str(cfg), '?')}), MI355X",
         "#",
-        "# command (repo root, GPU box):",
+        "# command (repo root):",
         f"#   rocprofv3 --kernel-trace --stats -d {kt_dir} -o {out_name} -- \\",
         f"#       python3 -u bench.py {bench_args}",
         "# durations in microseconds over every dispatch of the run (warm-up, timed steps and",
@@ -146,7 +146,7 @@ def traffic(fetch_dir: str, write_dir: str, cfetch_dir: str, cwrite_dir: str, cf
     lines = [
         f"# HBM traffic per launch -- {_label(cfg)} ({WORKLOADS.get(str(cfg), '?')}), MI355X",
         "#",
-        "# commands (repo root, GPU box), one counter per pass:",
+        "# commands (repo root), one counter per pass:",
         f"#   rocprofv3 --pmc FETCH_SIZE -d {fetch_dir} -o f -- python3 -u bench.py {bench_args}",
         f"#   rocprofv3 --pmc WRITE_SIZE -d {write_dir} -o w -- python3 -u bench.py {bench_args}",
         "# calibration: the same counters on bench.py --copy-calibration (1 GiB device copies):",
@@ -181,7 +181,7 @@ def insts(sq_dir: str, kt_dir: str, cfg: str, bench_args: str = "") -> str:
     lines = [
         f"# SQ instruction counters per dispatch -- {_label(cfg)} ({WORKLOADS.get(str(cfg), '?')}), MI355X",
         "#",
-        "# command (repo root, GPU box), one pass:",
+        "# command (repo root), one pass:",
         f"#   rocprofv3 --pmc {' '.join(INST_COUNTERS)} -d {sq_dir} -o sq -- \\",
         f"#       python3 -u bench.py {bench_args}",
         "# instructions issued per MFMA: SQ_INSTS_VALU as counted (whether it includes the",
