@@ -184,6 +184,9 @@ std::tuple<Tensor, Tensor, Tensor> qkv_rope(const Tensor& qkv_in, const Tensor& 
 
 Tensor qkv_rope_backward(const Tensor& dq_in, const Tensor& dk_in, const Tensor& dv_in,
                          const Tensor& cos_in, const Tensor& sin_in, int64_t pos0) {
+  for (const Tensor* t : {&dq_in, &dk_in, &dv_in})
+    TORCH_CHECK_VALUE(t->dim() == 4, "expected a 4-D [B, H, T, D] gradient, got shape ",
+                      t->sizes());
   need_gpu(dq_in, dk_in, dv_in, cos_in, sin_in);
   const c10::DeviceGuard guard(dq_in.device());
   const int64_t B = dq_in.size(0), H = dq_in.size(1), T = dq_in.size(2), D = dq_in.size(3);

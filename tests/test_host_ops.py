@@ -220,3 +220,13 @@ def test_overwriting_token_inputs_needs_the_words_too():
                        link_rows=[np.ones((1, 1), dtype=np.uint64)])
     with pytest.raises(RuntimeError, match="q_bits and kv_bits are needed"):
         lists.build((torch.zeros(1, 128, dtype=torch.int32), None, None))
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+@pytest.mark.parametrize("shape", [(1, 2, 128, 64, 1), (2, 128, 64)])
+def test_rope_backward_refuses_gradients_of_other_ranks(which, shape):
+    t = [torch.zeros(1, 2, 128, 64, dtype=torch.bfloat16) for _ in range(3)]
+    t[which] = torch.zeros(shape, dtype=torch.bfloat16)
+    cs = torch.zeros(128, 32)
+    with pytest.raises(ValueError, match="4-D"):
+        _lib.host().qkv_rope_backward(*t, cs, cs, 0)
