@@ -69,10 +69,10 @@ typedef struct t2t_tensor {
  *   kv_bits_off int32[Bm][nt]: bitmap slots of a tile row: partial tile
  *       (r, c) uses slot kv_bits_off[r] + c, and distinct partial tiles must
  *       get distinct slots (no other slot is read: a full tile has none, and a
- *       row without partial tiles needs no valid offset).  t2t_mask_meta writes b nt (nt + 1) / 2 +
- *       r (r + 1) / 2, the tile's position in the lower triangle, which is
- *       distinct only because its masks are causal (every partial tile has
- *       c <= r); a caller filling the tables for a mask with partial tiles
+ *       row without partial tiles needs no valid offset).  t2t_mask_meta
+ *       writes b nt (nt + 1) / 2 + r (r + 1) / 2, the tile's position in the
+ *       lower triangle, which is distinct only because its masks are causal
+ *       (every partial tile has c <= r); a caller filling the tables for a mask with partial tiles
  *       above the diagonal uses b nt^2 + r nt (one slot per tile);
  *   q_bits_slot int32[Bm][nt][nt]: bitmap slot of the i-th partial tile of a
  *       column (entries past q_num unspecified);
